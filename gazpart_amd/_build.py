@@ -13,17 +13,29 @@ OUT = os.path.join(HERE, "libgazpart_gpu.so")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
-    "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
+    "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
     # packed FP32 instructions are kept out of the generated code
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
 
 
 def build(verbose: bool = False) -> str:
-    cmd = [HIPCC, *FLAGS, *SRCS, *LIBS, "-o", OUT + ".tmp"]
-    if verbose:
-        print(" ".join(cmd), file=sys.stderr)
-    r = subprocess.run(cmd, capture_output=True, text=True)
+    # one object a source, side by side, then the link
+    objs = [os.path.join(HERE, os.path.basename(s)[:-4] + ".o") for s in SRCS]
+    cmds = [[HIPCC, *FLAGS, "-c", s, "-o", o] for s, o in zip(SRCS, objs)]
+    procs = []
+    for c in cmds:
+        if verbose:
+            print(" ".join(c), file=sys.stderr)
+        procs.append(subprocess.Popen(c, stderr=subprocess.PIPE, text=True))
+    errs = [p.communicate()[1] for p in procs]
+    for p, e in zip(procs, errs):
+        if p.returncode != 0:
+            raise RuntimeError(f"hipcc failed:\n{e[-4000:]}")
+    link = [HIPCC, "--offload-arch=gfx950", "-shared", *objs, *LIBS, "-o", OUT + ".tmp"]
+    r = subprocess.run(link, capture_output=True, text=True)
+    for o in objs:
+        os.remove(o)
     if r.returncode != 0:
         raise RuntimeError(f"hipcc failed:\n{r.stderr[-4000:]}")
     os.replace(OUT + ".tmp", OUT)

@@ -14,30 +14,41 @@
 
 namespace gpfft {
 
-// E and the radices of the lengths that have a plan: few passes (each
-// exchange is a trip through LDS) with at most 20 values a thread, so that
-// three lines fit in a thread's registers.
-template <int N> struct Plan { static constexpr bool ok = false; };
-#define GP_FFT_PLAN(N_, E_, ...)                                             \
-  template <> struct Plan<N_> {                                              \
+// E and the radices of the lengths that have a plan.  K = 0: kernels that
+// hold one line, few passes (each exchange is a trip through LDS).  K = 1:
+// kernels that hold three lines and their own work beside, fewer values a
+// thread where the length allows, so that several wavefronts fit on a SIMD
+// (256: 8 values leave room for one or two).
+template <int N, int K> struct Plan { static constexpr bool ok = false; };
+#define GP_FFT_PLAN(N_, K_, E_, ...)                                         \
+  template <> struct Plan<N_, K_> {                                          \
     static constexpr bool ok = true;                                         \
     static constexpr int N = N_, E = E_, T = N_ / E_;                        \
-    static constexpr int rad[4] = {__VA_ARGS__};                             \
+    static constexpr int rad[7] = {__VA_ARGS__};                             \
   }
-GP_FFT_PLAN(32, 8, 8, 4, 1, 1);
-GP_FFT_PLAN(48, 12, 12, 4, 1, 1);
-GP_FFT_PLAN(64, 8, 8, 8, 1, 1);
-GP_FFT_PLAN(80, 20, 10, 4, 2, 1);
-GP_FFT_PLAN(96, 12, 12, 4, 2, 1);
-GP_FFT_PLAN(100, 10, 10, 10, 1, 1);
-GP_FFT_PLAN(128, 8, 8, 4, 4, 1);
-GP_FFT_PLAN(144, 12, 12, 12, 1, 1);
-GP_FFT_PLAN(160, 20, 10, 4, 4, 1);
-GP_FFT_PLAN(192, 12, 12, 4, 4, 1);
-GP_FFT_PLAN(256, 8, 8, 8, 4, 1);
-GP_FFT_PLAN(320, 20, 10, 4, 4, 2);
-GP_FFT_PLAN(384, 12, 12, 4, 4, 2);
-GP_FFT_PLAN(512, 8, 8, 8, 8, 1);
+#define GP_FFT_BOTH(N_, E_, ...)                                             \
+  GP_FFT_PLAN(N_, 0, E_, __VA_ARGS__);                                       \
+  GP_FFT_PLAN(N_, 1, E_, __VA_ARGS__)
+GP_FFT_PLAN(32, 0, 8, 8, 4);
+GP_FFT_PLAN(32, 1, 4, 4, 4, 2);
+GP_FFT_BOTH(48, 12, 12, 4);
+GP_FFT_PLAN(64, 0, 8, 8, 8);
+GP_FFT_PLAN(64, 1, 4, 4, 4, 4);
+GP_FFT_BOTH(80, 10, 10, 2, 2, 2);
+GP_FFT_BOTH(96, 12, 12, 4, 2);
+GP_FFT_BOTH(100, 10, 10, 10);
+GP_FFT_PLAN(128, 0, 8, 8, 4, 4);
+GP_FFT_PLAN(128, 1, 4, 4, 4, 4, 2);
+GP_FFT_BOTH(144, 12, 12, 12);
+GP_FFT_BOTH(160, 10, 10, 2, 2, 2, 2);
+GP_FFT_BOTH(192, 12, 12, 4, 4);
+GP_FFT_PLAN(256, 0, 8, 8, 8, 4);
+GP_FFT_PLAN(256, 1, 4, 4, 4, 4, 4);
+GP_FFT_BOTH(320, 10, 10, 2, 2, 2, 2, 2);
+GP_FFT_BOTH(384, 12, 12, 4, 4, 2);
+GP_FFT_PLAN(512, 0, 8, 8, 8, 8);
+GP_FFT_PLAN(512, 1, 4, 4, 4, 4, 4, 2);
+#undef GP_FFT_BOTH
 #undef GP_FFT_PLAN
 
 __device__ __forceinline__ double2 cadd(double2 a, double2 b) { return {a.x + b.x, a.y + b.y}; }
@@ -50,25 +61,27 @@ template <int DIR> __device__ __forceinline__ double2 rot(double2 a) {
   return DIR > 0 ? double2{-a.y, a.x} : double2{a.y, -a.x};
 }
 
-// cos(2 pi k / r) and sin(2 pi k / r) at compile time: the angle folded into
-// an eighth of the circle (integers), then the Taylor series
-constexpr double series(double x, bool sine) {
-  double term = sine ? x : 1.0, sum = term;
-  for (int i = sine ? 2 : 1; i < 30; i += 2) {
-    term *= -x * x / (double)(i * (i + 1));
-    sum += term;
-  }
-  return sum;
+// cos of an angle in degrees, of the angles that radices 3, 5, 8, 10 and 12
+// have, to the last bit (a constant that is one bit off is off in every
+// transform of a run: 1e-14 after 40 steps)
+constexpr double cos_deg(int d) {
+  d = d % 360;
+  if (d < 0) d += 360;
+  if (d > 180) d = 360 - d;
+  if (d > 90) return -cos_deg(180 - d);
+  return d == 0    ? 1.0
+         : d == 18 ? 0.95105651629515357212
+         : d == 30 ? 0.86602540378443864676
+         : d == 36 ? 0.80901699437494742410
+         : d == 45 ? 0.70710678118654752440
+         : d == 54 ? 0.58778525229247312917
+         : d == 60 ? 0.5
+         : d == 72 ? 0.30901699437494742410
+                   : 0.0;   // 90
 }
-constexpr double PI2 = 6.283185307179586476925;
-constexpr double cosk(int k, int r) {
-  k %= r;
-  if (2 * k > r) k = r - k;                                  // cos is even
-  if (4 * k > r) return -cosk(r - 2 * k, 2 * r);             // pi - angle
-  if (8 * k > r) return series(PI2 * (double)(r - 4 * k) / (double)(4 * r), true);
-  return series(PI2 * (double)k / (double)r, false);
-}
-constexpr double sink(int k, int r) { return cosk(4 * k + 3 * r, 4 * r); }   // cos(angle - pi/2)
+// cos and sin of 2 pi k / r, 360 k divisible by r
+constexpr double cosk(int k, int r) { return cos_deg(360 * k / r); }
+constexpr double sink(int k, int r) { return cos_deg(360 * k / r - 90); }
 
 // R-point transforms of registers, in place, natural order
 template <int R, int DIR> struct Dft;
@@ -164,26 +177,31 @@ template <int DIR> struct Dft<8, DIR> : DftAB<2, 4, DIR> {};
 template <int DIR> struct Dft<10, DIR> : DftAB<2, 5, DIR> {};
 template <int DIR> struct Dft<12, DIR> : DftAB<3, 4, DIR> {};
 
+// lines in the registers of a thread
+template <int N, int K> using Lines = double2 (*)[Plan<N, K>::E];
+
 // NC lines of length N in the registers of thread t of their T threads;
 // tw[k] = exp(-2 pi i k / N).  DIR -1 forward, +1 backward, unnormalised.
 // X exchanges: X::put(c, index, value), X::get(c, index), X::ready(c)
 // between the puts and the gets of line c, X::again(c) before the puts of
 // line c (after the gets of earlier ones).
-template <int N, int DIR, int NC, int P, int NS, typename X>
-__device__ __forceinline__ void fft_pass(double2 (*v)[Plan<N>::E], X& x, const double2* tw, int t) {
-  using PL = Plan<N>;
+template <int N, int K, int DIR, int NC, int P, int NS, typename X>
+__device__ __forceinline__ void fft_pass(Lines<N, K> v, X& x, const double2* tw, int t) {
+  using PL = Plan<N, K>;
   constexpr int E = PL::E, T = PL::T, R = PL::rad[P], B = E / R;
   static_assert(B * R == E, "radix divides the values of a thread");
 #pragma unroll
   for (int b = 0; b < B; ++b) {
     double2 w[R];
     if constexpr (NS > 1) {
-      // w^r, r = 1..R-1, from one table entry
+      // every factor from the table: powers formed by multiplication cost a
+      // decimal digit over a run's transforms
       const int q = (t + T * b) % NS;
-      w[1] = tw[q * (N / (NS * R))];
-      if (DIR > 0) w[1].y = -w[1].y;
 #pragma unroll
-      for (int r = 2; r < R; ++r) w[r] = cmul(w[r / 2], w[r - r / 2]);
+      for (int r = 1; r < R; ++r) {
+        w[r] = tw[q * r * (N / (NS * R))];
+        if (DIR > 0) w[r].y = -w[r].y;
+      }
     }
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
@@ -214,12 +232,12 @@ __device__ __forceinline__ void fft_pass(double2 (*v)[Plan<N>::E], X& x, const d
 #pragma unroll
       for (int m = 0; m < E; ++m) v[c][m] = x.get(c, t + T * m);
     }
-    fft_pass<N, DIR, NC, P + 1, NS * R>(v, x, tw, t);
+    fft_pass<N, K, DIR, NC, P + 1, NS * R>(v, x, tw, t);
   }
 }
-template <int N, int DIR, int NC, typename X>
-__device__ __forceinline__ void fft(double2 (*v)[Plan<N>::E], X& x, const double2* tw, int t) {
-  fft_pass<N, DIR, NC, 0, 1>(v, x, tw, t);
+template <int N, int K, int DIR, int NC, typename X>
+__device__ __forceinline__ void fft(Lines<N, K> v, X& x, const double2* tw, int t) {
+  fft_pass<N, K, DIR, NC, 0, 1>(v, x, tw, t);
 }
 
 }  // namespace gpfft

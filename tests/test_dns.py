@@ -344,3 +344,33 @@ def test_gpu_reuse_spectral_differs_by_rounding_only(forcing):
         out.append(d.velocity())
     assert np.abs(out[1] - out[0]).max() <= 1e-12 * np.abs(out[0]).max()
     assert not np.array_equal(out[0], u0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [36, 48, 80, 96, 100, 128, 144])
+@pytest.mark.parametrize("reuse", [False, True])
+def test_gpu_lengths_match_oracle(n, reuse):
+    """Transform lengths of every radix mix (and one that takes the library's
+    transforms): velocity, vorticity and EPS_FLU after three steps of a
+    nonlinear field with energy in the filter's taper.  1e-11 of the largest
+    magnitude, as the other lengths above: rounding of a transform is
+    1e-16 log2(n^3), a step has seven, the steps amplify it by CFL < 1."""
+    from gazpart_amd.dns import Dns
+    u0 = random_velocity(n, n / 10.0, 50 + n)
+    nu, dt, ns = 0.01, 0.1 / n, 3
+    d = Dns(n, L2PI, nu, dt, reuse_spectral=reuse)
+    d.set_velocity(u0)
+    w0 = d.vorticity()
+    s = D.DnsRef(n, L2PI, nu, dt)
+    s.set_velocity(u0)
+    wr = D.btran(s.vorticity(), n)
+    assert np.abs(w0 - wr).max() <= 1e-11 * np.abs(wr).max()
+    d.step(ns)
+    for _ in range(ns):
+        s.step()
+    u = d.velocity()
+    assert np.abs(u - s.u).max() <= 1e-11 * np.abs(s.u).max()
+    w, wr = d.vorticity(), D.btran(s.vorticity(), n)
+    assert np.abs(w - wr).max() <= 1e-11 * np.abs(wr).max()
+    assert abs(d.info()["eps"] - s.eps) <= 1e-11 * s.eps
+    assert not np.array_equal(u, u0)
