@@ -58,6 +58,7 @@
 
 #include "../../include/gazpart_gpu.h"
 #include "gp_fft.h"
+#include "gp_xfer.h"
 
 namespace gpdns {
 
@@ -783,6 +784,7 @@ struct gp_dns {
   rocfft_plan fwd = nullptr, bwd = nullptr;
   rocfft_execution_info info = nullptr;
   void* work = nullptr;
+  gpx::Xfer xf;            // transfers with the caller's memory
   bool have_u = false;
   double eps = 0.0;
   // forcing: modes in the reference's loop order, amplitudes (host), the
@@ -1115,6 +1117,7 @@ int gp_dns_destroy(gp_dns* d) {
   for (void* b : bufs)
     if (b) hipFree(b);
   if (d->fpin) hipHostFree(d->fpin);
+  d->xf.release();
   if (d->st) hipStreamDestroy(d->st);
   delete d;
   return GP_OK;
@@ -1124,7 +1127,7 @@ const char* gp_dns_error_string(const gp_dns* d) { return d ? d->err.c_str() : "
 
 int gp_dns_set_velocity(gp_dns* d, const double* uvw) {
   if (!d || !uvw) return GP_ERR_ARG;
-  DCHK(hipMemcpyAsync(d->u, uvw, 3 * d->g.nr * sizeof(double), hipMemcpyHostToDevice, d->st));
+  DCHK(d->xf.h2d(d->u, uvw, 3 * (size_t)d->g.nr * sizeof(double), d->st));
   // the spectral state of this velocity (for gp_dns_get_vorticity / bind)
   if (d->tw) {
     with_passes(d->g.n, [&](auto ps) { ps.spectral(d); });
@@ -1147,8 +1150,7 @@ int gp_dns_get_velocity(gp_dns* d, double* uvw) {
     d->err = "no velocity (gp_dns_set_velocity)";
     return GP_ERR_STATE;
   }
-  DCHK(hipMemcpyAsync(uvw, d->u, 3 * d->g.nr * sizeof(double), hipMemcpyDeviceToHost, d->st));
-  DCHK(hipStreamSynchronize(d->st));
+  DCHK(d->xf.d2h(uvw, d->u, 3 * (size_t)d->g.nr * sizeof(double), d->st));
   return GP_OK;
 }
 
@@ -1173,8 +1175,7 @@ int gp_dns_get_vorticity(gp_dns* d, double* w) {
   }
   int rc;
   if ((rc = vorticity_dev(d))) return rc;
-  DCHK(hipMemcpyAsync(w, d->z, 3 * d->g.nr * sizeof(double), hipMemcpyDeviceToHost, d->st));
-  DCHK(hipStreamSynchronize(d->st));
+  DCHK(d->xf.d2h(w, d->z, 3 * (size_t)d->g.nr * sizeof(double), d->st));
   return GP_OK;
 }
 

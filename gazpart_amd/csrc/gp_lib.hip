@@ -36,6 +36,7 @@
 #include "gp_io.h"
 #include "gp_mlp.h"
 #include "gp_scan.h"
+#include "gp_xfer.h"
 
 namespace gp {
 
@@ -223,7 +224,6 @@ template <typename FT, int S> struct Row<FT, S, 1> {
     for (int i = 0; i < S; ++i) v[i] = p[i];
   }
 };
-
 // INTERP_LAG3 / INTERP_LAG4 of all six fields at once (interp_lag3.f90:
 // 119-290, interp_lag4.f90:84-312).  The field carries ghost planes in x as
 // well (index period n, the reference's x wrap of interp_lag3.f90:132-154),
@@ -1983,26 +1983,60 @@ __global__ void k_pos_of_id(PState<VT> p, int* pos, int np) {
   if (i < np) pos[p.id[i]] = i;
 }
 
+// The state crosses to the host and back in chunks of consecutive reference
+// indices: per chunk of m particles seven rows of doubles (x y z qa qb qc
+// qd), then six of the velocities' type (u v w ox oy oz), so that the mixed
+// form moves 80 bytes a particle instead of 104 (the workers of gp_xfer.h
+// convert on the host, which rounds as the device does).
 template <typename VT>
-__global__ void k_gather_out(PState<VT> p, double* out, int np) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= np) return;
-  double st[13];
-  load_state(p, i, st);
-  const int id = p.id[i];
-  for (int c = 0; c < 13; ++c) out[(long long)c * np + id] = st[c];
+__global__ __launch_bounds__(BLOCK) void k_gather_chunk(PState<VT> p,
+                                                        const int* __restrict__ pos_of_id, int i0,
+                                                        int m, double* __restrict__ out) {
+  const int k = blockIdx.x * BLOCK + threadIdx.x;
+  if (k >= m) return;
+  const int s = pos_of_id[i0 + k];
+  VT* __restrict__ v = reinterpret_cast<VT*>(out + 7 * (size_t)m);
+  out[k] = p.x[s];
+  out[(size_t)m + k] = p.y[s];
+  out[2 * (size_t)m + k] = p.z[s];
+  out[3 * (size_t)m + k] = p.qa[s];
+  out[4 * (size_t)m + k] = p.qb[s];
+  out[5 * (size_t)m + k] = p.qc[s];
+  out[6 * (size_t)m + k] = p.qd[s];
+  v[k] = p.u[s];
+  v[(size_t)m + k] = p.v[s];
+  v[2 * (size_t)m + k] = p.w[s];
+  v[3 * (size_t)m + k] = p.ox[s];
+  v[4 * (size_t)m + k] = p.oy[s];
+  v[5 * (size_t)m + k] = p.oz[s];
 }
 
+// the other way, with a row of species indices after the velocities
 template <typename VT>
-__global__ void k_scatter_in(PState<VT> p, const double* in, const int* sp,
-                             const Species* __restrict__ spec, int np) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= np) return;
-  double st[13];
-  for (int c = 0; c < 13; ++c) st[c] = in[(long long)c * np + i];
-  store_state(p, i, st);
-  p.sp[i] = sp[i];
-  p.rm[i] = float_up(spec[sp[i]].rmax);
+__global__ __launch_bounds__(BLOCK) void k_scatter_chunk(PState<VT> p,
+                                                         const double* __restrict__ in,
+                                                         const Species* __restrict__ spec, int i0,
+                                                         int m) {
+  const int k = blockIdx.x * BLOCK + threadIdx.x;
+  if (k >= m) return;
+  const int i = i0 + k;
+  const VT* __restrict__ v = reinterpret_cast<const VT*>(in + 7 * (size_t)m);
+  const int sid = reinterpret_cast<const int*>(v + 6 * (size_t)m)[k];
+  p.x[i] = in[k];
+  p.y[i] = in[(size_t)m + k];
+  p.z[i] = in[2 * (size_t)m + k];
+  p.qa[i] = in[3 * (size_t)m + k];
+  p.qb[i] = in[4 * (size_t)m + k];
+  p.qc[i] = in[5 * (size_t)m + k];
+  p.qd[i] = in[6 * (size_t)m + k];
+  p.u[i] = v[k];
+  p.v[i] = v[(size_t)m + k];
+  p.w[i] = v[2 * (size_t)m + k];
+  p.ox[i] = v[3 * (size_t)m + k];
+  p.oy[i] = v[4 * (size_t)m + k];
+  p.oz[i] = v[5 * (size_t)m + k];
+  p.sp[i] = sid;
+  p.rm[i] = float_up(spec[sid].rmax);
   p.id[i] = i;
   p.grp[i] = 0;
 }
@@ -2105,6 +2139,13 @@ struct gp_ctx {
   bool pipe_prev = false;
   int64_t batch_fallbacks = 0;  // gated seeded solves redone in the last gp_contact_batch
   double* scratch = nullptr;    // this device's copy of the gp_interph_noalloc staging
+  // transfers with the caller's memory, and the device scratch of the calls
+  // that need some for their own duration (device_scratch)
+  gpx::Xfer xf;
+  char* dscr = nullptr;
+  size_t dscr_n = 0;
+  // the sizes that the particle and grid buffers were allocated for
+  int alloc_np = 0, alloc_nbox = 0, alloc_nbrick = 0, alloc_scan_np = 0;
   // level-2 statistics: u - mean at the origin of each correlation slot,
   // 3 x np doubles by reference index (allocated when a slot starts)
   double* lag_u0[GP_NLGR] = {};
@@ -2289,6 +2330,43 @@ static int dalloc(gp_ctx* ctx, T** p, size_t count) {
     ctx->err = std::string("hipMalloc failed: ") + hipGetErrorString(e);
     return GP_ERR_NOMEM;
   }
+  return GP_OK;
+}
+
+// device memory for the duration of one call, kept between calls up to
+// DSCR_KEEP bytes (an allocation and its release cost more than the kernels of
+// a small call, and the release waits for the device)
+constexpr size_t DSCR_KEEP = (size_t)64 << 20;
+
+struct DeviceScratch {
+  char* p = nullptr;
+  bool own = false;
+  ~DeviceScratch() {
+    if (own && p) (void)hipFree(p);
+  }
+};
+
+static int device_scratch(gp_ctx* ctx, size_t bytes, DeviceScratch& d) {
+  if (bytes > DSCR_KEEP) {
+    d.own = true;
+    const hipError_t e = hipMalloc((void**)&d.p, bytes);
+    if (e != hipSuccess) {
+      d.p = nullptr;
+      ctx->err = std::string("HIP error: ") + hipGetErrorString(e) + " (device scratch)";
+      return GP_ERR_HIP;
+    }
+    return GP_OK;
+  }
+  if (bytes > ctx->dscr_n) {
+    HIPCHK(hipStreamSynchronize(ctx->st));
+    if (ctx->dscr) (void)hipFree(ctx->dscr);
+    ctx->dscr = nullptr;
+    ctx->dscr_n = 0;
+    const size_t n = std::min(DSCR_KEEP, bytes + bytes / 2);
+    HIPCHK(hipMalloc((void**)&ctx->dscr, n));
+    ctx->dscr_n = n;
+  }
+  d.p = ctx->dscr;
   return GP_OK;
 }
 
@@ -2629,6 +2707,12 @@ constexpr size_t TILE_LDS_MAX = 65536;
 
 static int ensure_grid_buffers(gp_ctx* ctx) {
   const CellGrid& g = ctx->g;
+  // the sizes of the last call: the buffers stand (nothing reads what an
+  // earlier set of particles left in them)
+  if (ctx->alloc_nbox == g.nbox && ctx->alloc_nbrick == ctx->bg.n &&
+      ctx->alloc_scan_np == ctx->np && ctx->scan_scr)
+    return GP_OK;
+  ctx->alloc_nbox = 0;
   int rc;
   if ((rc = dalloc(ctx, &ctx->cnt, (size_t)g.nbox))) return rc;
   if ((rc = dalloc(ctx, &ctx->off, (size_t)g.nbox + 1))) return rc;
@@ -2639,6 +2723,9 @@ static int ensure_grid_buffers(gp_ctx* ctx) {
   if (ctx->scan_scr) hipFree(ctx->scan_scr);
   ctx->scan_scr = nullptr;
   HIPCHK(hipMalloc(&ctx->scan_scr, (size_t)sc * sizeof(long long)));
+  ctx->alloc_nbox = g.nbox;
+  ctx->alloc_nbrick = ctx->bg.n;
+  ctx->alloc_scan_np = ctx->np;
   return GP_OK;
 }
 
@@ -2739,6 +2826,8 @@ int gp_destroy(gp_ctx* ctx) {
     if (b) hipFree(b);
   for (double* b : ctx->lag_u0)
     if (b) hipFree(b);
+  if (ctx->dscr) hipFree(ctx->dscr);
+  ctx->xf.release();
   for (auto& e : ctx->ev)
     if (e) hipEventDestroy(e);
   drop_graph(ctx);
@@ -2795,7 +2884,11 @@ int gp_bind_field(gp_ctx* ctx, const double* field) {
   const size_t nref = (size_t)6 * n * n4 * n4;
   double* dref = nullptr;
   HIPCHK(hipMalloc((void**)&dref, nref * sizeof(double)));
-  HIPCHK(hipMemcpyAsync(dref, field, nref * sizeof(double), hipMemcpyHostToDevice, ctx->st));
+  const hipError_t e = ctx->xf.h2d(dref, field, nref * sizeof(double), ctx->st);
+  if (e != hipSuccess) {
+    hipFree(dref);
+    HIPCHK(e);
+  }
   const int rc = bind_field_dev(ctx, dref);
   hipFree(dref);
   return rc;
@@ -2898,9 +2991,93 @@ int gp_set_species(gp_ctx* ctx, int nspec, const double* rows) {
   return GP_OK;
 }
 
+}  // extern "C"
+
+// the rows of the state a chunk holds, in the order k_gather_chunk writes them
+static const int STATE_ROW[13] = {0, 1, 2, 6, 7, 8, 9, 3, 4, 5, 10, 11, 12};
+
+// particles of one chunk: enough for all workers, within a buffer
+static int state_chunk(const gp_ctx* ctx, size_t row, int& n) {
+  n = gpx::Xfer::workers((size_t)ctx->np * row);
+  const size_t m = ((size_t)ctx->np + n - 1) / n;
+  return (int)std::min(gpx::XFER_CHUNK / row, (m + 255) / 256 * 256);
+}
+
+// the caller's state to buffer 0 (asynchronous on the stream where it returns)
+template <typename VT>
+static hipError_t send_state(gp_ctx* ctx, const double* state, const int* species) {
+  const size_t np = (size_t)ctx->np, row = 7 * sizeof(double) + 6 * sizeof(VT) + sizeof(int);
+  int n;
+  const int ch = state_chunk(ctx, row, n);
+  hipError_t e = ctx->xf.reserve(n, (size_t)ch * row, true);
+  if (e != hipSuccess) return e;
+  auto p = pstate<VT>(ctx, 0);
+  return gpx::Xfer::run(n, ((long long)np + ch - 1) / ch, [&](int b, long long q) {
+    gpx::Xfer& x = ctx->xf;
+    hipError_t r = q >= n ? hipEventSynchronize(x.ev[b]) : hipSuccess;   // the buffer's last chunk
+    if (r != hipSuccess) return r;
+    const size_t i0 = (size_t)q * ch, m = std::min<size_t>(ch, np - i0);
+    double* d = (double*)x.pin[b];
+    VT* v = (VT*)(d + 7 * m);
+    for (int c = 0; c < 7; ++c)
+      std::memcpy(d + c * m, state + STATE_ROW[c] * np + i0, m * sizeof(double));
+    for (int c = 0; c < 6; ++c) {
+      const double* src = state + STATE_ROW[7 + c] * np + i0;
+      VT* dst = v + c * m;
+      for (size_t k = 0; k < m; ++k) dst[k] = (VT)src[k];
+    }
+    std::memcpy(v + 6 * m, species + i0, m * sizeof(int));
+    r = hipMemcpyAsync(x.dev[b], x.pin[b], m * row, hipMemcpyHostToDevice, ctx->st);
+    if (r != hipSuccess) return r;
+    hipLaunchKernelGGL(k_scatter_chunk<VT>, dim3(nblk((long long)m)), dim3(BLOCK), 0, ctx->st, p,
+                       (const double*)x.dev[b], (const Species*)ctx->spec, (int)i0, (int)m);
+    r = hipGetLastError();
+    return r == hipSuccess ? hipEventRecord(x.ev[b], ctx->st) : r;
+  });
+}
+
+// the current state to the caller, in reference order
+template <typename VT>
+static hipError_t fetch_state(gp_ctx* ctx, double* state) {
+  const size_t np = (size_t)ctx->np, row = 7 * sizeof(double) + 6 * sizeof(VT);
+  int n;
+  const int ch = state_chunk(ctx, row, n);
+  hipError_t e = ctx->xf.reserve(n, (size_t)ch * row, true);
+  if (e != hipSuccess) return e;
+  auto p = pstate<VT>(ctx, ctx->cur);
+  hipLaunchKernelGGL(k_pos_of_id<VT>, dim3(nblk(ctx->np)), dim3(BLOCK), 0, ctx->st, p,
+                     ctx->pos_of_id, ctx->np);
+  if ((e = hipGetLastError()) != hipSuccess) return e;
+  return gpx::Xfer::run(n, ((long long)np + ch - 1) / ch, [&](int b, long long q) {
+    gpx::Xfer& x = ctx->xf;
+    const size_t i0 = (size_t)q * ch, m = std::min<size_t>(ch, np - i0);
+    hipLaunchKernelGGL(k_gather_chunk<VT>, dim3(nblk((long long)m)), dim3(BLOCK), 0, ctx->st, p,
+                       (const int*)ctx->pos_of_id, (int)i0, (int)m, (double*)x.dev[b]);
+    hipError_t r = hipGetLastError();
+    if (r == hipSuccess)
+      r = hipMemcpyAsync(x.pin[b], x.dev[b], m * row, hipMemcpyDeviceToHost, ctx->st);
+    if (r == hipSuccess) r = hipEventRecord(x.ev[b], ctx->st);
+    if (r == hipSuccess) r = hipEventSynchronize(x.ev[b]);
+    if (r != hipSuccess) return r;
+    const double* d = (const double*)x.pin[b];
+    const VT* v = (const VT*)(d + 7 * m);
+    for (int c = 0; c < 7; ++c)
+      std::memcpy(state + STATE_ROW[c] * np + i0, d + c * m, m * sizeof(double));
+    for (int c = 0; c < 6; ++c) {
+      const VT* src = v + c * m;
+      double* dst = state + STATE_ROW[7 + c] * np + i0;
+      for (size_t k = 0; k < m; ++k) dst[k] = (double)src[k];
+    }
+    return r;
+  });
+}
+
+extern "C" {
+
 int gp_set_particles(gp_ctx* ctx, int np, const double* state, const int* species) {
   if (!ctx || np < 1 || !state || !species) return GP_ERR_ARG;
   hipStreamSynchronize(ctx->st);
+  hipStreamSynchronize(ctx->st2);
   hipStreamSynchronize(ctx->st3);
   drop_graph(ctx);
   ctx->contacts_valid = false;
@@ -2918,78 +3095,76 @@ int gp_set_particles(gp_ctx* ctx, int np, const double* state, const int* specie
     return GP_ERR_STATE;
   }
   int max_sp = 0;
+  unsigned out = 0;   // one pass without a branch an element
   for (int i = 0; i < np; ++i) {
-    if (species[i] < 0 || species[i] >= ctx->nspec) {
-      ctx->err = "species index out of range at particle " + std::to_string(i);
-      return GP_ERR_ARG;
-    }
+    out |= (unsigned)((unsigned)species[i] >= (unsigned)ctx->nspec);
     max_sp = std::max(max_sp, species[i]);
   }
-  ctx->np = np;
-  ctx->max_sp = max_sp;
-  const size_t pb = pstate_bytes(np, ctx->mixed);
-  for (int k = 0; k < 2; ++k) {
-    if (ctx->pbuf[k]) hipFree(ctx->pbuf[k]);
-    ctx->pbuf[k] = nullptr;
-    HIPCHK(hipMalloc(&ctx->pbuf[k], pb));
+  if (out) {
+    int i = 0;
+    while (species[i] >= 0 && species[i] < ctx->nspec) ++i;
+    ctx->err = "species index out of range at particle " + std::to_string(i);
+    return GP_ERR_ARG;
   }
   int rc;
-  if ((rc = dalloc(ctx, &ctx->perm, (size_t)np))) return rc;
-  if ((rc = dalloc(ctx, &ctx->cell, (size_t)np))) return rc;
-  if ((rc = dalloc(ctx, &ctx->slot, (size_t)np))) return rc;
-  if ((rc = dalloc(ctx, &ctx->tkey, (size_t)np))) return rc;
-  if ((rc = dalloc(ctx, &ctx->sorted, (size_t)np))) return rc;
-  if ((rc = dalloc(ctx, &ctx->pcount, (size_t)np))) return rc;
-  if ((rc = dalloc(ctx, &ctx->poff, (size_t)np + 1))) return rc;
-  if ((rc = dalloc(ctx, &ctx->mark, (size_t)np))) return rc;
-  if ((rc = dalloc(ctx, &ctx->used, (size_t)np))) return rc;
-  if ((rc = dalloc(ctx, &ctx->pos_of_id, (size_t)np))) return rc;
-  if ((rc = dalloc(ctx, &ctx->brick, (size_t)np))) return rc;
-  if ((rc = dalloc(ctx, &ctx->bslot, (size_t)np))) return rc;
-  if ((rc = dalloc(ctx, &ctx->trav, (size_t)np))) return rc;
-  if ((rc = dalloc(ctx, &ctx->pos4, (size_t)np))) return rc;
-  if ((rc = dalloc(ctx, &ctx->csort, (size_t)np))) return rc;
-  if ((rc = dalloc(ctx, &ctx->gsort, (size_t)np))) return rc;
-  if ((rc = dalloc(ctx, &ctx->inlm, (size_t)np))) return rc;
-  if ((rc = dalloc(ctx, &ctx->plist, (size_t)np))) return rc;
-  if ((rc = dalloc(ctx, &ctx->inv, (size_t)np))) return rc;
-  if ((rc = dalloc(ctx, &ctx->ccount, (size_t)np))) return rc;
-  HIPCHK(hipMemset(ctx->inlm, 0, (size_t)np * sizeof(int)));
-  HIPCHK(hipMemset(ctx->ccount, 0, (size_t)np * sizeof(int)));
-  if (ctx->prm.tile > 0) {
-    if (ctx->mixed) {
-      if ((rc = dalloc(ctx, (float**)&ctx->flpre, (size_t)np * 6))) return rc;
-    } else {
-      if ((rc = dalloc(ctx, (double**)&ctx->flpre, (size_t)np * 6))) return rc;
+  // as many particles as before: every buffer stands
+  const bool keep = ctx->alloc_np == np && ctx->pbuf[0] && ctx->pbuf[1];
+  ctx->np = np;
+  ctx->max_sp = max_sp;
+  if (!keep) {
+    ctx->alloc_np = 0;
+    const size_t pb = pstate_bytes(np, ctx->mixed);
+    for (int k = 0; k < 2; ++k) {
+      if (ctx->pbuf[k]) hipFree(ctx->pbuf[k]);
+      ctx->pbuf[k] = nullptr;
+      HIPCHK(hipMalloc(&ctx->pbuf[k], pb));
     }
+    if ((rc = dalloc(ctx, &ctx->perm, (size_t)np))) return rc;
+    if ((rc = dalloc(ctx, &ctx->cell, (size_t)np))) return rc;
+    if ((rc = dalloc(ctx, &ctx->slot, (size_t)np))) return rc;
+    if ((rc = dalloc(ctx, &ctx->tkey, (size_t)np))) return rc;
+    if ((rc = dalloc(ctx, &ctx->sorted, (size_t)np))) return rc;
+    if ((rc = dalloc(ctx, &ctx->pcount, (size_t)np))) return rc;
+    if ((rc = dalloc(ctx, &ctx->poff, (size_t)np + 1))) return rc;
+    if ((rc = dalloc(ctx, &ctx->mark, (size_t)np))) return rc;
+    if ((rc = dalloc(ctx, &ctx->used, (size_t)np))) return rc;
+    if ((rc = dalloc(ctx, &ctx->pos_of_id, (size_t)np))) return rc;
+    if ((rc = dalloc(ctx, &ctx->brick, (size_t)np))) return rc;
+    if ((rc = dalloc(ctx, &ctx->bslot, (size_t)np))) return rc;
+    if ((rc = dalloc(ctx, &ctx->trav, (size_t)np))) return rc;
+    if ((rc = dalloc(ctx, &ctx->pos4, (size_t)np))) return rc;
+    if ((rc = dalloc(ctx, &ctx->csort, (size_t)np))) return rc;
+    if ((rc = dalloc(ctx, &ctx->gsort, (size_t)np))) return rc;
+    if ((rc = dalloc(ctx, &ctx->inlm, (size_t)np))) return rc;
+    if ((rc = dalloc(ctx, &ctx->plist, (size_t)np))) return rc;
+    if ((rc = dalloc(ctx, &ctx->inv, (size_t)np))) return rc;
+    if ((rc = dalloc(ctx, &ctx->ccount, (size_t)np))) return rc;
+    if (ctx->prm.tile > 0) {
+      if (ctx->mixed) {
+        if ((rc = dalloc(ctx, (float**)&ctx->flpre, (size_t)np * 6))) return rc;
+      } else {
+        if ((rc = dalloc(ctx, (double**)&ctx->flpre, (size_t)np * 6))) return rc;
+      }
+    }
+    if (ctx->prm.keep_fluid) {
+      if ((rc = dalloc(ctx, &ctx->flout, (size_t)np * 6))) return rc;
+    }
+    ctx->alloc_np = np;
   }
   ctx->flpre_valid = false;
-  if (ctx->prm.keep_fluid) {
-    if ((rc = dalloc(ctx, &ctx->flout, (size_t)np * 6))) return rc;
-  }
   if ((rc = ensure_grid_buffers(ctx))) return rc;
+  hipLaunchKernelGGL(k_fill<int>, dim3(nblk(np)), dim3(BLOCK), 0, ctx->st, ctx->inlm, 0,
+                     (long long)np);
+  hipLaunchKernelGGL(k_fill<int>, dim3(nblk(np)), dim3(BLOCK), 0, ctx->st, ctx->ccount, 0,
+                     (long long)np);
   hipLaunchKernelGGL(k_fill<long long>, dim3(nblk(np)), dim3(BLOCK), 0, ctx->st, ctx->mark,
                      (long long)LLONG_MAX, (long long)np);
   hipLaunchKernelGGL(k_fill<int>, dim3(nblk(np)), dim3(BLOCK), 0, ctx->st, ctx->used, 0,
                      (long long)np);
-  double* din = nullptr;
-  int* dsp = nullptr;
-  HIPCHK(hipMalloc((void**)&din, (size_t)np * 13 * sizeof(double)));
-  HIPCHK(hipMalloc((void**)&dsp, (size_t)np * sizeof(int)));
-  HIPCHK(hipMemcpyAsync(din, state, (size_t)np * 13 * sizeof(double), hipMemcpyHostToDevice,
-                        ctx->st));
-  HIPCHK(hipMemcpyAsync(dsp, species, (size_t)np * sizeof(int), hipMemcpyHostToDevice, ctx->st));
   ctx->cur = 0;
-  if (ctx->mixed)
-    hipLaunchKernelGGL(k_scatter_in<float>, dim3(nblk(np)), dim3(BLOCK), 0, ctx->st,
-                       pstate<float>(ctx, 0), din, dsp, ctx->spec, np);
-  else
-    hipLaunchKernelGGL(k_scatter_in<double>, dim3(nblk(np)), dim3(BLOCK), 0, ctx->st,
-                       pstate<double>(ctx, 0), din, dsp, ctx->spec, np);
-  HIPCHK(hipGetLastError());
+  HIPCHK(ctx->mixed ? send_state<float>(ctx, state, species)
+                    : send_state<double>(ctx, state, species));
   HIPCHK(hipStreamSynchronize(ctx->st));
-  hipFree(din);
-  hipFree(dsp);
   ctx->perm_identity = true;
   ctx->cells_valid = false;
   ctx->ngroups = 1;
@@ -3028,27 +3203,13 @@ int gp_set_groups(gp_ctx* ctx, int np, const int* group) {
 
 int gp_get_particles(gp_ctx* ctx, int np, double* state) {
   if (!ctx || !state || np != ctx->np) return GP_ERR_ARG;
-  double* dout = nullptr;
-  HIPCHK(hipMalloc((void**)&dout, (size_t)np * 13 * sizeof(double)));
-  if (ctx->mixed)
-    hipLaunchKernelGGL(k_gather_out<float>, dim3(nblk(np)), dim3(BLOCK), 0, ctx->st,
-                       pstate<float>(ctx, ctx->cur), dout, np);
-  else
-    hipLaunchKernelGGL(k_gather_out<double>, dim3(nblk(np)), dim3(BLOCK), 0, ctx->st,
-                       pstate<double>(ctx, ctx->cur), dout, np);
-  HIPCHK(hipGetLastError());
-  HIPCHK(hipMemcpyAsync(state, dout, (size_t)np * 13 * sizeof(double), hipMemcpyDeviceToHost,
-                        ctx->st));
-  HIPCHK(hipStreamSynchronize(ctx->st));
-  hipFree(dout);
+  if (np > 0) HIPCHK(ctx->mixed ? fetch_state<float>(ctx, state) : fetch_state<double>(ctx, state));
   return check_err(ctx);
 }
 
 int gp_get_fluid_at_particles(gp_ctx* ctx, int np, double* fl) {
   if (!ctx || !fl || np != ctx->np || !ctx->flout) return GP_ERR_ARG;
-  HIPCHK(hipMemcpyAsync(fl, ctx->flout, (size_t)np * 6 * sizeof(double), hipMemcpyDeviceToHost,
-                        ctx->st));
-  HIPCHK(hipStreamSynchronize(ctx->st));
+  HIPCHK(ctx->xf.d2h(fl, ctx->flout, (size_t)np * 6 * sizeof(double), ctx->st));
   return GP_OK;
 }
 
@@ -3107,11 +3268,9 @@ int gp_interph(gp_ctx* ctx, int scheme, int nint, const double* x, const double*
   int rc = interph_args(ctx, scheme, nint, comp);
   if (rc) return rc;
   if (nint == 0) return GP_OK;
-  double* d = nullptr;
-  HIPCHK(hipMalloc((void**)&d, (size_t)nint * 4 * sizeof(double)));
-  rc = interph_staged(ctx, scheme, nint, x, y, z, comp, out, d);
-  hipFree(d);
-  if (rc) return rc;
+  DeviceScratch d;
+  if ((rc = device_scratch(ctx, (size_t)nint * 4 * sizeof(double), d))) return rc;
+  if ((rc = interph_staged(ctx, scheme, nint, x, y, z, comp, out, (double*)d.p))) return rc;
   return check_err(ctx);
 }
 
@@ -3432,15 +3591,18 @@ static int ensure_lists(gp_ctx* ctx, unsigned long long need) {
     const unsigned long long cap = need + need / 4 + 1024;
     if ((rc = dalloc(ctx, &ctx->work, (size_t)cap))) return rc;
     if ((rc = dalloc(ctx, &ctx->lmwork, (size_t)cap))) return rc;
-    if ((rc = dalloc(ctx, &ctx->seeds, (size_t)cap * 2))) return rc;
+    // the network's seeds, where it seeds the solves
+    if (ctx->prm.lm_seed == 1 && (rc = dalloc(ctx, &ctx->seeds, (size_t)cap * 2))) return rc;
     ctx->work_cap = cap;
   }
   // solving ahead: lists of an eighth of the work capacity (the survivors
   // of both filters are a small part of the bounding-sphere survivors; a
-  // pair past the capacity is simply solved in its own step), tables of
+  // pair past the capacity is simply solved in its own step), at most four
+  // times the solves up to which solving ahead is on (early_on), tables of
   // twice that (a power of two), keys and list counts cleared
   const unsigned long long ecap =
-      std::min(ctx->work_cap, std::max<unsigned long long>(ctx->work_cap / 8, 65536));
+      std::min({ctx->work_cap, std::max<unsigned long long>(ctx->work_cap / 8, 65536),
+                4ull * 64ull * (unsigned long long)ctx->nsimd});
   if (ecap > ctx->ep_cap) {
     HIPCHK(hipStreamSynchronize(ctx->st3));
     drop_graph(ctx);
@@ -3637,14 +3799,17 @@ static int launch_contacts(gp_ctx* ctx) {
   return launch_contacts_solve<VT>(ctx);
 }
 
-// COLLISION with the list sizes read back from the device
+// COLLISION with the list sizes read back from the device; headroom: the lists
+// are sized for the steps that follow without such a read (at once: the
+// lists of a dense suspension are gigabytes, and allocating them for this
+// pass and then again for the next ones took as long again)
 template <typename VT>
-static int launch_collide(gp_ctx* ctx) {
+static int launch_collide(gp_ctx* ctx, bool headroom = false) {
   int rc;
   if ((rc = launch_sort_count<VT>(ctx))) return rc;
   // prefilter survivors <= candidates
-  if ((rc = ensure_lists(ctx, (unsigned long long)std::max<long long>(ctx->last_nclose, 1))))
-    return rc;
+  const unsigned long long n = (unsigned long long)std::max<long long>(ctx->last_nclose, 1);
+  if ((rc = ensure_lists(ctx, headroom ? 2ull * n + 4096ull : n))) return rc;
   if ((rc = launch_contacts<VT>(ctx))) return rc;
   ctx->contacts_valid = true;
   ctx->pipe_prev = false;
@@ -3850,7 +4015,7 @@ static int graph_steps(gp_ctx* ctx, int nsteps) {
     hipLaunchKernelGGL(k_fill<unsigned long long>, dim3(1), dim3(1), 0, ctx->st, ctx->d_cnt, 0ull,
                        1ll);
     if ((rc = launch_advance<VT>(ctx, true))) return rc;
-    if ((rc = launch_collide<VT>(ctx))) return rc;
+    if ((rc = launch_collide<VT>(ctx, true))) return rc;
     --nsteps;
     const unsigned long long need = 2ull * (unsigned long long)ctx->last_nclose + 4096ull;
     if ((rc = ensure_lists(ctx, need))) return rc;
@@ -3951,11 +4116,11 @@ int gp_collision_detection(gp_ctx* ctx, int64_t nclosemax, int* home, int* near_
                      ctx->sorted, ctx->cell, ctx->off, ctx->cnt, ctx->poff, id,
                      ctx->ngroups > 1 ? ctx->gsort : nullptr, dh, dn, ctx->np);
   HIPCHK(hipGetLastError());
-  HIPCHK(hipMemcpyAsync(home, dh, (size_t)total * sizeof(int), hipMemcpyDeviceToHost, ctx->st));
-  HIPCHK(hipMemcpyAsync(near_, dn, (size_t)total * sizeof(int), hipMemcpyDeviceToHost, ctx->st));
-  HIPCHK(hipStreamSynchronize(ctx->st));
+  hipError_t e = ctx->xf.d2h(home, dh, (size_t)total * sizeof(int), ctx->st);
+  if (e == hipSuccess) e = ctx->xf.d2h(near_, dn, (size_t)total * sizeof(int), ctx->st);
   hipFree(dh);
   hipFree(dn);
+  HIPCHK(e);
   return GP_OK;
 }
 
@@ -4117,7 +4282,7 @@ int gp_collision_advance(gp_ctx* ctx, int ncycle, double time, int ncycle_next) 
   if (!ctx->lists_sized) {
     // an eager pass sizes the lists with headroom; later calls then run
     // without host synchronisation
-    rc = ctx->mixed ? launch_collide<float>(ctx) : launch_collide<double>(ctx);
+    rc = ctx->mixed ? launch_collide<float>(ctx, true) : launch_collide<double>(ctx, true);
     if (rc) return rc;
     const unsigned long long need = 2ull * (unsigned long long)ctx->last_nclose + 4096ull;
     if ((rc = ensure_lists(ctx, need))) return rc;
@@ -4275,14 +4440,13 @@ int gp_particle_stats(gp_ctx* ctx, int nspec, int npoly, int ref_norm, double* o
   int rc = ready(ctx);
   if (rc) return rc;
   if (!out || nspec != ctx->nspec || npoly < 1 || nspec % npoly) return GP_ERR_ARG;
-  double *acc = nullptr, *mean = nullptr;
   const size_t na = (size_t)nspec * NSTP, nm = (size_t)nspec * 10;
-  if (hipMalloc((void**)&acc, na * sizeof(double)) != hipSuccess ||
-      hipMalloc((void**)&mean, nm * sizeof(double)) != hipSuccess) {
-    if (acc) hipFree(acc);
+  DeviceScratch ds;
+  if (device_scratch(ctx, (na + nm) * sizeof(double), ds)) {
     ctx->err = "particle statistics: out of device memory";
     return GP_ERR_NOMEM;
   }
+  double *acc = (double*)ds.p, *mean = acc + na;
   const unsigned grid = std::max(1u, std::min(nblk(ctx->np), 2048u));
   const unsigned sgrid = nblk(nspec);
   hipMemsetAsync(acc, 0, na * sizeof(double), ctx->st);
@@ -4304,11 +4468,7 @@ int gp_particle_stats(gp_ctx* ctx, int nspec, int npoly, int ref_norm, double* o
   hipLaunchKernelGGL(k_pstat_final, dim3(sgrid), dim3(BLOCK), 0, ctx->st, ctx->spec, acc,
                      (const double*)mean, nspec, npoly, ref_norm ? 1 : 0);
   hipError_t e = hipGetLastError();
-  if (e == hipSuccess) e = hipMemcpyAsync(out, acc, na * sizeof(double), hipMemcpyDeviceToHost,
-                                          ctx->st);
-  if (e == hipSuccess) e = hipStreamSynchronize(ctx->st);
-  hipFree(acc);
-  hipFree(mean);
+  if (e == hipSuccess) e = ctx->xf.d2h(out, acc, na * sizeof(double), ctx->st);
   if (e != hipSuccess) {
     ctx->err = std::string("particle statistics: ") + hipGetErrorString(e);
     return GP_ERR_HIP;
@@ -4468,16 +4628,13 @@ int gp_partfluid_stats(gp_ctx* ctx, int nspec, int npoly, int ref_norm, double* 
     c[2] = (2.0 / 9.0) * (rhop * (minax * minax)) / (ctx->prm.rhof * ctx->prm.visc) * fbeta;
     c[3] = r[GP_SP_GRAV];
   }
-  double *acc = nullptr, *dout = nullptr, *dpfc = nullptr;
   const size_t na = (size_t)nspec * NPFS;
-  if (hipMalloc((void**)&acc, na * sizeof(double)) != hipSuccess ||
-      hipMalloc((void**)&dout, na * sizeof(double)) != hipSuccess ||
-      hipMalloc((void**)&dpfc, pfc.size() * sizeof(double)) != hipSuccess) {
-    if (acc) hipFree(acc);
-    if (dout) hipFree(dout);
+  DeviceScratch ds;
+  if (device_scratch(ctx, (2 * na + pfc.size()) * sizeof(double), ds)) {
     ctx->err = "particle-fluid statistics: out of device memory";
     return GP_ERR_NOMEM;
   }
+  double *acc = (double*)ds.p, *dout = acc + na, *dpfc = dout + na;
   hipError_t e = hipMemcpyAsync(dpfc, pfc.data(), pfc.size() * sizeof(double),
                                 hipMemcpyHostToDevice, ctx->st);
   // MEAN_PARTFLUID_LOC(:,:,:) = ZERO (:114)
@@ -4495,12 +4652,7 @@ int gp_partfluid_stats(gp_ctx* ctx, int nspec, int npoly, int ref_norm, double* 
   hipLaunchKernelGGL(k_pfstat_final, dim3(nblk(nspec)), dim3(BLOCK), 0, ctx->st,
                      (const double*)acc, dout, nspec, npoly, ref_norm ? 1 : 0);
   if (e == hipSuccess) e = hipGetLastError();
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(out, dout, na * sizeof(double), hipMemcpyDeviceToHost, ctx->st);
-  if (e == hipSuccess) e = hipStreamSynchronize(ctx->st);
-  hipFree(acc);
-  hipFree(dout);
-  hipFree(dpfc);
+  if (e == hipSuccess) e = ctx->xf.d2h(out, dout, na * sizeof(double), ctx->st);
   if (e != hipSuccess) {
     ctx->err = std::string("particle-fluid statistics: ") + hipGetErrorString(e);
     return GP_ERR_HIP;
@@ -4513,11 +4665,12 @@ int gp_particle_pdf(gp_ctx* ctx, int nspec, double* out) {
   if (rc) return rc;
   if (!out || nspec != ctx->nspec) return GP_ERR_ARG;
   const size_t nh = (size_t)nspec * PDF_Q * GP_NPDF;
-  unsigned* hist = nullptr;
-  if (hipMalloc((void**)&hist, nh * sizeof(unsigned)) != hipSuccess) {
+  DeviceScratch ds;
+  if (device_scratch(ctx, nh * sizeof(unsigned), ds)) {
     ctx->err = "particle PDFs: out of device memory";
     return GP_ERR_NOMEM;
   }
+  unsigned* hist = (unsigned*)ds.p;
   HIPCHK(hipMemsetAsync(hist, 0, nh * sizeof(unsigned), ctx->st));
   const unsigned grid = std::max(1u, std::min(nblk(ctx->np), 1024u));
   if (ctx->mixed)
@@ -4528,10 +4681,7 @@ int gp_particle_pdf(gp_ctx* ctx, int nspec, double* out) {
                        pstate<double>(ctx, ctx->cur), ctx->np, nspec, hist);
   std::vector<unsigned> h(nh);
   hipError_t e = hipGetLastError();
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(h.data(), hist, nh * sizeof(unsigned), hipMemcpyDeviceToHost, ctx->st);
-  if (e == hipSuccess) e = hipStreamSynchronize(ctx->st);
-  hipFree(hist);
+  if (e == hipSuccess) e = ctx->xf.d2h(h.data(), hist, nh * sizeof(unsigned), ctx->st);
   if (e != hipSuccess) {
     ctx->err = std::string("particle PDFs: ") + hipGetErrorString(e);
     return GP_ERR_HIP;
@@ -4556,8 +4706,9 @@ int gp_lagrangian_origin(gp_ctx* ctx, int slot, int nspec, const double* mean) {
     ctx->err = "Lagrangian origin: out of device memory";
     return GP_ERR_NOMEM;
   }
-  double* dm = nullptr;
-  HIPCHK(hipMalloc((void**)&dm, 3 * (size_t)nspec * sizeof(double)));
+  DeviceScratch ds;
+  if ((rc = device_scratch(ctx, 3 * (size_t)nspec * sizeof(double), ds))) return rc;
+  double* dm = (double*)ds.p;
   HIPCHK(hipMemcpyAsync(dm, mean, 3 * (size_t)nspec * sizeof(double), hipMemcpyHostToDevice,
                         ctx->st));
   if (ctx->mixed)
@@ -4569,7 +4720,6 @@ int gp_lagrangian_origin(gp_ctx* ctx, int slot, int nspec, const double* mean) {
                        ctx->lag_u0[slot]);
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(ctx->st));
-  hipFree(dm);
   return check_err(ctx);
 }
 
@@ -4584,8 +4734,9 @@ int gp_lagrangian_corr(gp_ctx* ctx, int slot, int nspec, const double* mean, con
     return GP_ERR_STATE;
   }
   const size_t ns3 = 3 * (size_t)nspec;
-  double* d = nullptr;
-  HIPCHK(hipMalloc((void**)&d, (2 * ns3 + nspec) * sizeof(double)));
+  DeviceScratch ds;
+  if ((rc = device_scratch(ctx, (2 * ns3 + nspec) * sizeof(double), ds))) return rc;
+  double* d = (double*)ds.p;
   double *dm = d, *dn = d + ns3, *dout = d + ns3 + nspec;
   HIPCHK(hipMemcpyAsync(dm, mean, ns3 * sizeof(double), hipMemcpyHostToDevice, ctx->st));
   HIPCHK(hipMemcpyAsync(dn, npm, (size_t)nspec * sizeof(double), hipMemcpyHostToDevice, ctx->st));
@@ -4600,9 +4751,7 @@ int gp_lagrangian_corr(gp_ctx* ctx, int slot, int nspec, const double* mean, con
                        pstate<double>(ctx, ctx->cur), ctx->np, nspec, (const double*)dm,
                        (const double*)dn, (const double*)ctx->lag_u0[slot], dout);
   HIPCHK(hipGetLastError());
-  HIPCHK(hipMemcpyAsync(out, dout, ns3 * sizeof(double), hipMemcpyDeviceToHost, ctx->st));
-  HIPCHK(hipStreamSynchronize(ctx->st));
-  hipFree(d);
+  HIPCHK(ctx->xf.d2h(out, dout, ns3 * sizeof(double), ctx->st));
   return check_err(ctx);
 }
 
