@@ -170,6 +170,25 @@ __device__ __forceinline__ int block_index(int xcd_remap) {
   return (b & 7) * per + (b >> 3);
 }
 
+// The advance's workgroup order in the reference's cell order (x fastest, then
+// y, then z): the particles of a z layer are cut into eight y blocks, one
+// for each XCD, and every XCD goes through its own y block layer by layer.
+// Layers are taken as equally full (the order is a permutation of the
+// workgroups whatever the particles do; how well the caches do depends on
+// it).  layers = 0: block_index.
+struct LayerMap {
+  int nb = 0;       // workgroups with work
+  int layers = 0;   // z layers of cells
+  int per = 0;      // workgroups launched for each (layer, y block), nb's share rounded up
+};
+__device__ __forceinline__ int layer_block(const LayerMap& lm, int xcd_remap) {
+  if (!lm.layers) return block_index(xcd_remap);
+  const int b = blockIdx.x, y = b & 7, t = b >> 3, j = t % lm.per, z = t / lm.per;
+  const long long k = 8ll * z + y, n = 8ll * lm.layers;
+  const int lo = (int)(k * lm.nb / n), hi = (int)((k + 1) * lm.nb / n);
+  return lo + j < hi ? lo + j : lm.nb;   // nb: nothing to do
+}
+
 __device__ __forceinline__ long long node_index(int n4, int i, int j, int k) {
   return ((long long)(k + 1) * n4 + (j + 1)) * n4 + (i + 1);
 }
@@ -661,8 +680,8 @@ __global__ __launch_bounds__(BLOCK) void k_advance(
     PState<VT> dst, const int* __restrict__ perm, int np, CellGrid g, int* __restrict__ cell,
     int* __restrict__ slot, int* __restrict__ cnt, BrickGrid bg, int* __restrict__ brick,
     int* __restrict__ bslot, int* __restrict__ bcnt, unsigned* err, unsigned long long* nwall,
-    double* __restrict__ flout, int xcd, const int* __restrict__ skip) {
-  const int i = block_index(xcd) * BLOCK + threadIdx.x;
+    double* __restrict__ flout, int xcd, LayerMap lm, const int* __restrict__ skip) {
+  const int i = layer_block(lm, xcd) * BLOCK + threadIdx.x;
   if (i >= np) return;
   const int s = perm ? perm[i] : i;
   if (skip && skip[s]) return;
@@ -3413,13 +3432,23 @@ static void launch_advance_kernel(gp_ctx* ctx, hipStream_t st, const int* perm, 
     return;
   }
   unsigned nb = nblk(np);
+  // y blocks per XCD where a layer's y block fills four workgroups or more: at
+  // 8e6 particles on 512^3 (12 of them) the FP32 advance takes 2620 us against
+  // 2804 in plain order, at 1e6 on 256^3 (2.5) 344 against 338
+  LayerMap lm;
+  if (!xcd && perm && perm != ctx->trav && nb >= 32u * (unsigned)ctx->g.nz) {
+    lm.nb = (int)nb;
+    lm.layers = ctx->g.nz;
+    lm.per = (int)((nb + 8u * ctx->g.nz - 1) / (8u * ctx->g.nz));
+    nb = 8u * (unsigned)lm.layers * (unsigned)lm.per;
+  }
   if (xcd) nb = (nb + 7) / 8 * 8;
   const dim3 gr(nb), bl(BLOCK);
 #define GP_ADV(FT, CT, S)                                                                        \
   hipLaunchKernelGGL((k_advance<FT, VT, CT, S>), gr, bl, 0, st, ctx->sp, (const FT*)ctx->field, \
                      ctx->spec, ps, pd, perm, np, ctx->g, cell, ctx->slot, ctx->cnt, ctx->bg,    \
                      ctx->brick, ctx->bslot, bcnt, ctx->d_err, ctx->d_cnt + 0, ctx->flout, xcd,  \
-                     skip)
+                     lm, skip)
   if (ctx->mixed) {
     if (ctx->prm.interp_scheme == 3) GP_ADV(float, float, 4);
     else GP_ADV(float, float, 5);

@@ -1,10 +1,12 @@
-"""Transfers between the caller's memory and the device: the state comes back
-as it was given whatever the number of particles (one chunk, several, a last
-chunk of one particle; fewer or more particles than before in the same
-context).
+"""Transfers between the caller's memory and the device, and the advance's
+workgroup order: the state comes back as it was given whatever the number of
+particles (one chunk, several, a last chunk of one particle; fewer or more
+particles than before in the same context), and no order of the workgroups
+changes a result.
 
 No tolerance: FP64 values are copied, the mixed form keeps the velocities and
-spins as float32 (round to nearest)."""
+spins as float32 (round to nearest), and the order of independent particles
+leaves every bit."""
 import numpy as np
 import pytest
 
@@ -46,3 +48,44 @@ def test_state_round_trip(G, prec):
     with pytest.raises(G.GpError):
         ctx.set_particles(st, np.full(5, 3, dtype=np.int32))
     np.testing.assert_array_equal(ctx.get_particles(), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,scheme", [(24, 3), (33, 4)])
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("np_,nz", [(163_840, 20), (170_003, 20), (20_011, 16)])
+def test_workgroup_order_changes_no_result(G, n, scheme, prec, np_, nz):
+    """nz layers of collision cells: the layer order of the advance's
+    workgroups (four workgroups or more a layer and y block; the last case has
+    fewer and keeps the plain order), against one range per XCD"""
+    from gazpart_amd import workload as W
+    wl = W.build_workload("order", n, np_, scheme=scheme, apr=2.0, emaj_dx=0.02, st=1.0, seed=np_)
+    out = []
+    for xcd in (0, 1):
+        ctx = G.Context(wl.n, wl.L, wl.visc, wl.rhof, wl.dtime, scheme=scheme, precision=prec,
+                        dpmax=wl.L / (2.0 * nz + 0.5), xcd_remap=xcd, graph=2)
+        ctx.bind_field(wl.field)
+        ctx.set_species(wl.species)
+        ctx.set_particles(wl.state, wl.species_id)
+        ctx.step(4)
+        out.append(ctx.get_particles())
+    np.testing.assert_array_equal(out[0], out[1])
+    assert not np.array_equal(out[0], wl.state)
+
+
+def test_layer_order_takes_every_workgroup_once():
+    """the order itself, restated: every workgroup exactly once"""
+    for nb in (32, 33, 100, 157, 274, 3907):
+        for layers in (1, 2, 3, 7, nb // 32):
+            if layers < 1 or nb < 32 * layers:
+                continue
+            per = (nb + 8 * layers - 1) // (8 * layers)
+            seen = []
+            for b in range(8 * layers * per):
+                y, t = b & 7, b >> 3
+                j, z = t % per, t // per
+                k, n = 8 * z + y, 8 * layers
+                lo, hi = k * nb // n, (k + 1) * nb // n
+                if lo + j < hi:
+                    seen.append(lo + j)
+            assert sorted(seen) == list(range(nb)), (nb, layers)
