@@ -243,6 +243,15 @@ template <typename FT, int S> struct Row<FT, S, 1> {
     for (int i = 0; i < S; ++i) v[i] = p[i];
   }
 };
+// one component of an interleaved row
+template <typename FT, int S> struct RowOne {
+  FT v[S];
+  __device__ __forceinline__ void load(const FT* __restrict__ p) {
+#pragma unroll
+    for (int i = 0; i < S; ++i) v[i] = p[6 * i];
+  }
+};
+
 // INTERP_LAG3 / INTERP_LAG4 of all six fields at once (interp_lag3.f90:
 // 119-290, interp_lag4.f90:84-312).  The field carries ghost planes in x as
 // well (index period n, the reference's x wrap of interp_lag3.f90:132-154),
@@ -294,7 +303,7 @@ template <int S> constexpr int stencil_lo() { return (S == 4) ? -1 : -2; }
 // FP32 and 900 -> 460 us FP64 (8e6 on 512^3: 2968 -> 2113 us); k_advance
 // 817 -> 602 us FP64, 350 us FP32 as before (its arithmetic beside), the
 // listed advance 240 -> 96 us FP64.
-template <typename FT, typename CT, int S, int NC, typename RowAt>
+template <typename FT, typename CT, int S, int NC, typename RowT = Row<FT, S, NC>, typename RowAt>
 __device__ __forceinline__ void stencil_sum(const Stencil<CT, S>& w, const RowAt& row,
                                             CT out[NC]) {
   CT acc[NC], fz[S];
@@ -309,7 +318,7 @@ __device__ __forceinline__ void stencil_sum(const Stencil<CT, S>& w, const RowAt
     for (int c = 0; c < NC; ++c) sy[c] = CT(0);
 #pragma unroll
     for (int j2 = 0; j2 < 4; j2 += 2) {
-      Row<FT, S, NC> r[2];
+      RowT r[2];
       r[0].load(row(j2, kz));
       r[1].load(row(j2 + 1, kz));
       __builtin_amdgcn_sched_barrier(0);
@@ -567,6 +576,10 @@ __global__ void k_field_prep_planar(const double* __restrict__ u, const double* 
   for (int c = 0; c < 3; ++c) out[t * 6 + 3 + c] = (FT)(vscale * w[c * nr + src]);
 }
 
+// one component at given points: reads that component's values alone (a row
+// spans the same cache lines, but a lane asks for 4-5 values of it instead of
+// 24-30, and the address path takes one lane's line a clock): 100,000 points
+// on 128^3 FP64 96 -> 62 us
 template <typename FT, typename CT, int S>
 __global__ __launch_bounds__(BLOCK) void k_interph(const FT* __restrict__ f, int n, double dx,
                                                    const double* __restrict__ x,
@@ -576,13 +589,22 @@ __global__ __launch_bounds__(BLOCK) void k_interph(const FT* __restrict__ f, int
                                                    unsigned* err) {
   int p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= nint) return;
-  CT v[6];
-  if (!gather6<FT, CT, S>(f, n, dx, x[p], y[p], z[p], v)) {
+  Stencil<CT, S> w;
+  if (!stencil_at<CT, S>(n, dx, x[p], y[p], z[p], w)) {
     atomicOr(err, EB_INTERP_RANGE);
     out[p] = 0.0;
     return;
   }
-  out[p] = (double)v[comp];
+  constexpr int lo = stencil_lo<S>();
+  const int n4 = n + 4;
+  CT v[1];
+  stencil_sum<FT, CT, S, 1, RowOne<FT, S>>(
+      w,
+      [&](int jy, int kz) {
+        return f + node_index(n4, w.i0 + lo, w.j0 + lo + jy, w.k0 + lo + kz) * 6 + comp;
+      },
+      v);
+  out[p] = (double)v[0];
 }
 
 template <typename FT, typename CT, int S>
@@ -2645,8 +2667,11 @@ __global__ __launch_bounds__(BLOCK) void k_pfstat(PState<VT> p, const double* __
     for (int c = 0; c < 6; ++c) uf[c] = fl[(long long)c * np + id];
     double e[NPFS];
     partfluid_entries(R, up, om, uf, pfc + 4 * (size_t)sp, visc, rhof, e);
-    double* dst = lds ? s_acc + sp * NPFS : acc + (size_t)sp * NPFS;
-    for (int k = 0; k < NPFS; ++k) atomicAdd(dst + k, e[k]);
+    // apart, so that the LDS sums are LDS atomics and not flat ones
+    if (lds)
+      for (int k = 0; k < NPFS; ++k) atomicAdd(&s_acc[sp * NPFS + k], e[k]);
+    else
+      for (int k = 0; k < NPFS; ++k) atomicAdd(&acc[(size_t)sp * NPFS + k], e[k]);
   }
   if (lds) {
     __syncthreads();
