@@ -1281,6 +1281,49 @@ __device__ __forceinline__ int table_get(const unsigned long long* keys, const i
   return -1;
 }
 
+// One slot per lane that asks in each of NL lists, one atomic a list and
+// workgroup (every thread of the workgroup calls it; sh is its scratch).  The
+// counters are single words that all workgroups add to, and such atomics go
+// through one after the other: per wavefront they set the time of the filter
+// of a dense suspension (2e6 particles in 5 % by
+// volume, 5e5 solves of 2.5e6 pairs: 737 -> 400 us).
+template <int NL> struct BlockAppend {
+  unsigned n[NL][BLOCK / 64];
+  unsigned long long base[NL];
+};
+template <int NL>
+__device__ __forceinline__ void block_append(BlockAppend<NL>& sh, const bool (&want)[NL],
+                                             unsigned long long* const (&count)[NL],
+                                             unsigned long long (&at)[NL]) {
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  unsigned below[NL];
+#pragma unroll
+  for (int l = 0; l < NL; ++l) {
+    const unsigned long long m = __ballot(want[l]);
+    below[l] = (unsigned)__popcll(m & ((1ull << lane) - 1ull));
+    if (lane == 0) sh.n[l][wv] = (unsigned)__popcll(m);
+  }
+  __syncthreads();
+  if (threadIdx.x < NL) {
+    unsigned t = 0;
+#pragma unroll
+    for (int w = 0; w < BLOCK / 64; ++w) t += sh.n[threadIdx.x][w];
+    unsigned long long* c = nullptr;
+#pragma unroll
+    for (int l = 0; l < NL; ++l) c = (int)threadIdx.x == l ? count[l] : c;
+    sh.base[threadIdx.x] = t ? atomicAdd(c, (unsigned long long)t) : 0ull;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int l = 0; l < NL; ++l) {
+    unsigned before = 0;
+#pragma unroll
+    for (int w = 0; w < BLOCK / 64; ++w) before += w < wv ? sh.n[l][w] : 0u;
+    at[l] = sh.base[l] + before + below[l];
+  }
+  __syncthreads();   // the scratch is free for the next call
+}
+
 // one slot per lane that asks, one atomic per wavefront
 __device__ __forceinline__ unsigned long long wave_append(bool want, unsigned long long* count) {
   const int lane = threadIdx.x & 63;
@@ -1304,11 +1347,11 @@ __global__ __launch_bounds__(BLOCK) void k_pw_filter(
     const unsigned long long* nwork, unsigned long long cap, double L, int use_pw,
     WorkRec* __restrict__ lm, unsigned long long* nlm, int* __restrict__ flag,
     int* __restrict__ plist, unsigned long long* nplist, SideClear sc, EarlyTab et) {
+  __shared__ BlockAppend<3> sh;
   side_clear(sc);
   const unsigned long long nw = min(*nwork, cap);
-  const int lane = threadIdx.x & 63;
-  // the loop bound is uniform over the workgroup, so every lane of a
-  // wavefront takes part in each ballot
+  // the loop bound is uniform over the workgroup, so every lane of it takes
+  // part in each append
   for (unsigned long long b0 = (unsigned long long)blockIdx.x * blockDim.x; b0 < nw;
        b0 += (unsigned long long)gridDim.x * blockDim.x) {
     const unsigned long long w = b0 + threadIdx.x;
@@ -1355,32 +1398,15 @@ __global__ __launch_bounds__(BLOCK) void k_pw_filter(
         solve = false;
       }
     }
-    // one atomic per wavefront: ballot + prefix
-    const unsigned long long m = __ballot(solve);
-    if (m) {
-      const int leader = __ffsll((long long)m) - 1;
-      unsigned long long base = 0;
-      if (lane == leader) base = atomicAdd(nlm, (unsigned long long)__popcll(m));
-      base = __shfl(base, leader);
-      if (solve) lm[base + __popcll(m & ((1ull << lane) - 1ull))] = r;
-    }
-    // flag (once) and list the particles of the solves, whose advance of the
-    // next step waits for this step's collisions
-    if (flag) {
-      const bool ci = pass && atomicExch(&flag[r.i], 1) == 0;
-      const bool cj = pass && atomicExch(&flag[r.j], 1) == 0;
-      const unsigned long long mi = __ballot(ci), mj = __ballot(cj);
-      const int ni = __popcll(mi), nt = ni + __popcll(mj);
-      if (nt) {
-        const int leader = __ffsll((long long)(mi | mj)) - 1;
-        unsigned long long base = 0;
-        if (lane == leader) base = atomicAdd(nplist, (unsigned long long)nt);
-        base = __shfl(base, leader);
-        const unsigned long long below = (1ull << lane) - 1ull;
-        if (ci) plist[base + __popcll(mi & below)] = r.i;
-        if (cj) plist[base + ni + __popcll(mj & below)] = r.j;
-      }
-    }
+    // the solve list, and the particles of the solves flagged (once) and
+    // listed: their advance of the next step waits for this step's collisions
+    const bool ci = flag && pass && atomicExch(&flag[r.i], 1) == 0;
+    const bool cj = flag && pass && atomicExch(&flag[r.j], 1) == 0;
+    unsigned long long at[3];
+    block_append<3>(sh, {solve, ci, cj}, {nlm, nplist, nplist}, at);
+    if (solve) lm[at[0]] = r;
+    if (ci) plist[at[1]] = r.i;
+    if (cj) plist[at[2]] = r.j;
   }
 }
 

@@ -89,3 +89,48 @@ def test_layer_order_takes_every_workgroup_once():
                 if lo + j < hi:
                     seen.append(lo + j)
             assert sorted(seen) == list(range(nb)), (nb, layers)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("np_,cells", [(300, 14), (3_000, 14), (3_000, 9), (20_000, 12)])
+def test_collision_pass_matches_the_candidate_list(G, np_, cells):
+    """The filters, the solve list and the one-collision pass against the
+    materialised candidate list solved pair by pair: cells of less and of
+    more than a particle on average, contacts from none (their rounds in one
+    workgroup, from the second pass on) to hundreds.  Lists and counts are
+    whole numbers: equal."""
+    from gazpart_amd import contacts as CT
+    from gazpart_amd import workload as W
+    L = 2.0 * np.pi
+    a = L / (4.0 * cells + 0.5)
+    sp = W.species_spheroid(a, 2.0, 500.0)[None, :]
+    sid = np.zeros(np_, dtype=np.int32)
+    st = W.random_particles(np_, L, a, 5)
+    st[3:6] = np.random.default_rng(np_).standard_normal((3, np_))
+    ctx = G.Context(16, L, 0.01, 1.0, 1e-4, dpmax=2.0 * a)
+    ctx.set_species(sp)
+    ctx.bind_field(np.zeros((6, 20, 20, 16)))
+    ctx.set_particles(st, sid)
+    for rep in range(3):
+        st = ctx.get_particles()
+        home, near = ctx.collision_detection_connectivity()
+        flag, e1, e2, cn, _ = ctx.ellipsoid_contact_detection(home, near)
+        qd = CT.decision_quantities(st, sp, sid, L, home, near, e1, e2, cn)
+        hit = CT.contact_of(flag, qd)
+        used, want = np.zeros(np_ + 1, dtype=bool), []
+        for h, n in zip(home[hit], near[hit]):
+            want.append(not (used[h] or used[n]))
+            if want[-1]:
+                used[h] = used[n] = True
+        ctx.collision()
+        s = ctx.stats()
+        assert s["nclose"] == len(home)
+        h, n, r = ctx.contacts()
+        np.testing.assert_array_equal(h, home[hit])
+        np.testing.assert_array_equal(n, near[hit])
+        np.testing.assert_array_equal(r, want)
+        assert s["ncollision"] == sum(want)
+        assert want or rep or np_ < 1_000
+        after = ctx.get_particles()
+        moved = (after != st).any(axis=0)
+        np.testing.assert_array_equal(np.nonzero(moved)[0] + 1, np.nonzero(used)[0])
