@@ -1127,8 +1127,11 @@ __device__ __forceinline__ void min_image(const PState<VT>& p, int i, int j, dou
 constexpr int PF_STAGE = 1024;
 
 // GROUPED: several ensembles (gsort given), a variant of its own so that
-// the plain test keeps its registers
-template <bool GROUPED>
+// the plain test keeps its registers.  DENSE: cells of a particle or more on
+// average, whose further members are read three at a time (one trip to the
+// caches for three tests): 2e6 particles in 5 % by volume 610 -> 490 us; in
+// sparse cells (1e6 in 1e-3: 0.14 a cell) it took 84 us against 80.
+template <bool GROUPED, bool DENSE = false>
 __global__ __launch_bounds__(BLOCK) void k_prefilter(
     CellGrid g, const float4* __restrict__ pos4, const int* __restrict__ sorted,
     const int* __restrict__ csort, const int* __restrict__ off, const int* __restrict__ cnt,
@@ -1191,7 +1194,17 @@ __global__ __launch_bounds__(BLOCK) void k_prefilter(
       for (int r = 0; r < 14; ++r) {
         if (slo[r] < sup[r]) {
           test(first[r], slo[r]);
-          for (int t = slo[r] + 1; t < sup[r]; ++t) test(pos4[t], t);
+          if (!DENSE) {
+            for (int t = slo[r] + 1; t < sup[r]; ++t) test(pos4[t], t);
+          } else {
+            for (int t = slo[r] + 1; t < sup[r]; t += 3) {
+              const float4 a = pos4[t], b = pos4[min(t + 1, sup[r] - 1)],
+                           d = pos4[min(t + 2, sup[r] - 1)];
+              test(a, t);
+              if (t + 1 < sup[r]) test(b, t + 1);
+              if (t + 2 < sup[r]) test(d, t + 2);
+            }
+          }
         }
       }
     } else {
@@ -3772,7 +3785,8 @@ static int launch_contacts_filter(gp_ctx* ctx, bool list_lm, bool clear_bins = f
                        ctx->work, c + 1, ctx->work_cap, c + 11, ctx->d_err, np,
                        ctx->prm.xcd_remap);
   else
-    hipLaunchKernelGGL(k_prefilter<false>, dim3(xcd_grid(ctx, np)), dim3(BLOCK), 0, ctx->st,
+    hipLaunchKernelGGL((np >= ctx->g.nbox ? k_prefilter<false, true> : k_prefilter<false, false>),
+                       dim3(xcd_grid(ctx, np)), dim3(BLOCK), 0, ctx->st,
                        ctx->g, ctx->pos4, ctx->sorted, ctx->csort, ctx->off, ctx->cnt,
                        (const int*)nullptr, ctx->prm.L, prefilter_tol(ctx), ctx->prm.prefilter,
                        ctx->work, c + 1, ctx->work_cap, c + 11, ctx->d_err, np,
