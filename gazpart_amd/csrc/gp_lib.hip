@@ -1799,18 +1799,12 @@ __device__ __forceinline__ int ld_relaxed(int* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// rounds 2, 3, ... over the contacts still undecided (one workgroup)
-__global__ __launch_bounds__(GREEDY_BLOCK) void k_greedy_rounds(
-    const ActiveRec* __restrict__ act, const unsigned long long* nact, unsigned long long acap,
-    long long* mark, int* used, unsigned char* __restrict__ status,
-    const unsigned long long* left, unsigned long long* rounds_out) {
-  if (*left == 0) {
-    if (threadIdx.x == 0) *rounds_out += 1ull;
-    return;
-  }
-  const long long na = (long long)min(*nact, acap);
+// rounds over the contacts still undecided, one workgroup; returns how many
+__device__ __forceinline__ int greedy_rounds_wg(const ActiveRec* __restrict__ act, long long na,
+                                                long long* mark, int* used,
+                                                unsigned char* __restrict__ status) {
   __shared__ int s_left;
-  int rounds = 1;
+  int rounds = 0;
   for (;;) {
     if (threadIdx.x == 0) s_left = 0;
     for (long long a = threadIdx.x; a < na; a += blockDim.x) {
@@ -1848,6 +1842,34 @@ __global__ __launch_bounds__(GREEDY_BLOCK) void k_greedy_rounds(
     __syncthreads();
     if (nleft == 0) break;
   }
+  return rounds;
+}
+
+// rounds 2, 3, ... (returns at once when nothing is undecided)
+__global__ __launch_bounds__(GREEDY_BLOCK) void k_greedy_rounds(
+    const ActiveRec* __restrict__ act, const unsigned long long* nact, unsigned long long acap,
+    long long* mark, int* used, unsigned char* __restrict__ status,
+    const unsigned long long* left, unsigned long long* rounds_out) {
+  int rounds = 1;
+  if (*left != 0)
+    rounds += greedy_rounds_wg(act, (long long)min(*nact, acap), mark, used, status);
+  if (threadIdx.x == 0) *rounds_out += (unsigned long long)rounds;
+}
+
+// every round in one workgroup, one launch instead of four, where the last
+// known count of solves (which bounds the contacts and, unlike them, does not
+// depend on the velocities) is at most GREEDY_FEW; any number is right.
+// Bound by the launches: 1e4 particles on 64^3 (some ten contacts) 13.7 us in
+// four launches, 5.0 us in one (a pass of 64 steps 13.2 -> 12.1 ms).
+// Thousands of contacts want more than one workgroup.
+constexpr unsigned long long GREEDY_FEW = 4096;
+__global__ __launch_bounds__(GREEDY_BLOCK) void k_greedy_few(
+    const ActiveRec* __restrict__ act, const unsigned long long* nact, unsigned long long acap,
+    long long* mark, int* used, unsigned char* __restrict__ status,
+    unsigned long long* rounds_out) {
+  const long long na = (long long)min(*nact, acap);
+  for (long long a = threadIdx.x; a < na; a += blockDim.x) status[a] = 0;   // its own contacts
+  const int rounds = na ? greedy_rounds_wg(act, na, mark, used, status) : 1;
   if (threadIdx.x == 0) *rounds_out += (unsigned long long)rounds;
 }
 
@@ -2311,6 +2333,7 @@ struct gp_ctx {
   int ep_par = 0;
   bool ep_step = false;            // this step solves ahead
   unsigned long long last_nlm = 0; // last known count of contact solves
+  bool nlm_known = false;
 };
 
 // ---------------------------------------------------------------------------
@@ -3857,14 +3880,19 @@ static int launch_contacts_solve(gp_ctx* ctx) {
                        c + 4, c + 7, ctx->d_err);
   }
   mark(ctx, 3);
-  hipLaunchKernelGGL(k_greedy_mark, dim3(GREEDY_GRID), dim3(BLOCK), 0, ctx->st, ctx->act, c + 2,
-                     ctx->act_cap, ctx->mark);
-  hipLaunchKernelGGL(k_greedy_accept, dim3(GREEDY_GRID), dim3(BLOCK), 0, ctx->st, ctx->act,
-                     c + 2, ctx->act_cap, ctx->mark, ctx->used, ctx->act_status);
-  hipLaunchKernelGGL(k_greedy_drop, dim3(GREEDY_GRID), dim3(BLOCK), 0, ctx->st, ctx->act, c + 2,
-                     ctx->act_cap, ctx->mark, ctx->used, ctx->act_status, c + 8);
-  hipLaunchKernelGGL(k_greedy_rounds, dim3(1), dim3(GREEDY_BLOCK), 0, ctx->st, ctx->act, c + 2,
-                     ctx->act_cap, ctx->mark, ctx->used, ctx->act_status, c + 8, c + 6);
+  if (ctx->nlm_known && ctx->last_nlm <= GREEDY_FEW) {
+    hipLaunchKernelGGL(k_greedy_few, dim3(1), dim3(GREEDY_BLOCK), 0, ctx->st, ctx->act, c + 2,
+                       ctx->act_cap, ctx->mark, ctx->used, ctx->act_status, c + 6);
+  } else {
+    hipLaunchKernelGGL(k_greedy_mark, dim3(GREEDY_GRID), dim3(BLOCK), 0, ctx->st, ctx->act, c + 2,
+                       ctx->act_cap, ctx->mark);
+    hipLaunchKernelGGL(k_greedy_accept, dim3(GREEDY_GRID), dim3(BLOCK), 0, ctx->st, ctx->act,
+                       c + 2, ctx->act_cap, ctx->mark, ctx->used, ctx->act_status);
+    hipLaunchKernelGGL(k_greedy_drop, dim3(GREEDY_GRID), dim3(BLOCK), 0, ctx->st, ctx->act, c + 2,
+                       ctx->act_cap, ctx->mark, ctx->used, ctx->act_status, c + 8);
+    hipLaunchKernelGGL(k_greedy_rounds, dim3(1), dim3(GREEDY_BLOCK), 0, ctx->st, ctx->act, c + 2,
+                       ctx->act_cap, ctx->mark, ctx->used, ctx->act_status, c + 8, c + 6);
+  }
   hipLaunchKernelGGL(k_greedy_impulse<VT>, dim3(GREEDY_GRID), dim3(BLOCK), 0, ctx->st, ps,
                      ctx->spec, ctx->act, c + 2, ctx->act_cap, ctx->used, ctx->act_status, c + 5,
                      ctx->d_err, ctx->ccount, cs.rec ? ctx->mark : nullptr);
@@ -4088,6 +4116,7 @@ static int capture_graph(gp_ctx* ctx) {
 // register budget; 4 queue behind them).  No effect on results.
 static void choose_lm_waves(gp_ctx* ctx, unsigned long long nlm) {
   ctx->last_nlm = nlm;
+  ctx->nlm_known = true;
   if (ctx->prm.lm_waves > 0) return;
   const unsigned long long lanes = (unsigned long long)ctx->nsimd * 64ull;
   ctx->lm_waves = ctx->nsimd * (nlm >= 4 * lanes ? 4 : nlm >= lanes ? 2 : 1);
