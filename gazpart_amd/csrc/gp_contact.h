@@ -115,6 +115,28 @@ struct Jet {
   double d[3];             // p1 - p2
 };
 
+// Sums of products here and below are written as fused operations: which
+// product is rounded by itself is then the same in every copy of the solve
+// (the fast run, the run with scaled sums, the seeded one), where the
+// compiler's choice hangs on the products that it happens to share.
+__device__ __forceinline__ double dot3(double e0, double e1, double e2, const double v[3]) {
+  return __builtin_fma(e2, v[2], __builtin_fma(e0, v[0], e1 * v[1]));
+}
+__device__ __forceinline__ void solve_symv(const Sym3& e, const double v[3], double o[3]) {
+  o[0] = dot3(e.xx, e.xy, e.xz, v);
+  o[1] = dot3(e.xy, e.yy, e.yz, v);
+  o[2] = dot3(e.xz, e.yz, e.zz, v);
+}
+// the same with v[2] = 0 (kept as a factor: it passes infinities on)
+__device__ __forceinline__ double dot30(double e0, double e1, double e2, const double v[3]) {
+  return __builtin_fma(e2, v[2], __builtin_fma(e1, v[1], e0 * v[0]));
+}
+__device__ __forceinline__ void solve_symv0(const Sym3& e, const double v[3], double o[3]) {
+  o[0] = dot30(e.xx, e.xy, e.xz, v);
+  o[1] = dot30(e.xy, e.yy, e.yz, v);
+  o[2] = dot30(e.xz, e.yz, e.zz, v);
+}
+
 // support of the normal cv(x) = (cos x0 cos x1, sin x0 cos x1, sin x1):
 // p1 = b1 + E1 cv / (2 l1), p2 = b2 - E2 cv / (2 l2); residuals
 // f_i = (p1 - p2)_i^2
@@ -123,10 +145,10 @@ __device__ __forceinline__ void support(const ContactPair& cp, const double x[2]
   sincos(x[0], &s.s0, &s.c0);
   sincos(x[1], &s.s1, &s.c1);
   const double cv[3] = {s.c0 * s.c1, s.s0 * s.c1, s.s1};
-  symv(cp.E1, cv, s.t1);
-  symv(cp.E2, cv, s.t2);   // E2 (-cv) = -t2
-  s.l1 = sqrt(0.25 * (cv[0] * s.t1[0] + cv[1] * s.t1[1] + cv[2] * s.t1[2]));
-  s.l2 = sqrt(0.25 * (cv[0] * s.t2[0] + cv[1] * s.t2[1] + cv[2] * s.t2[2]));
+  solve_symv(cp.E1, cv, s.t1);
+  solve_symv(cp.E2, cv, s.t2);   // E2 (-cv) = -t2
+  s.l1 = sqrt(0.25 * dot3(s.t1[0], s.t1[1], s.t1[2], cv));
+  s.l2 = sqrt(0.25 * dot3(s.t2[0], s.t2[1], s.t2[2], cv));
   s.h1 = 1.0 / (2.0 * s.l1);
   s.h2 = 1.0 / (2.0 * s.l2);
   for (int i = 0; i < 3; ++i) {
@@ -154,12 +176,12 @@ __device__ __forceinline__ void fcn_j(const ContactPair& cp, const Jet& s, doubl
   const double g1[3] = {-s.c0 * s.s1, -s.s0 * s.s1, s.c1};
   const double k1 = 1.0 / (8.0 * s.l1 * s.l1 * s.l1), k2 = 1.0 / (8.0 * s.l2 * s.l2 * s.l2);
   double e1g0[3], e1g1[3], e2g0[3], e2g1[3];
-  symv(cp.E1, g0, e1g0); symv(cp.E1, g1, e1g1);
-  symv(cp.E2, g0, e2g0); symv(cp.E2, g1, e2g1);
-  const double t1g0 = s.t1[0] * g0[0] + s.t1[1] * g0[1] + s.t1[2] * g0[2];
-  const double t1g1 = s.t1[0] * g1[0] + s.t1[1] * g1[1] + s.t1[2] * g1[2];
-  const double t2g0 = s.t2[0] * g0[0] + s.t2[1] * g0[1] + s.t2[2] * g0[2];
-  const double t2g1 = s.t2[0] * g1[0] + s.t2[1] * g1[1] + s.t2[2] * g1[2];
+  solve_symv0(cp.E1, g0, e1g0); solve_symv(cp.E1, g1, e1g1);
+  solve_symv0(cp.E2, g0, e2g0); solve_symv(cp.E2, g1, e2g1);
+  const double t1g0 = dot30(s.t1[0], s.t1[1], s.t1[2], g0);
+  const double t1g1 = dot3(s.t1[0], s.t1[1], s.t1[2], g1);
+  const double t2g0 = dot30(s.t2[0], s.t2[1], s.t2[2], g0);
+  const double t2g1 = dot3(s.t2[0], s.t2[1], s.t2[2], g1);
   for (int i = 0; i < 3; ++i) {
     const double gd0 = s.h1 * e1g0[i] - k1 * s.t1[i] * t1g0 + s.h2 * e2g0[i] - k2 * s.t2[i] * t2g0;
     const double gd1 = s.h1 * e1g1[i] - k1 * s.t1[i] * t1g1 + s.h2 * e2g1[i] - k2 * s.t2[i] * t2g1;
@@ -173,9 +195,7 @@ __device__ __forceinline__ void fcn_j(const ContactPair& cp, const Jet& s, doubl
 __device__ __forceinline__ double pick(const double a[2], int l) { return l ? a[1] : a[0]; }
 
 // enorm (minpack_reduc.f90:180-232), MINPACK's scaled sums for
-// components that are tiny (<= rdwarf) or huge (>= rgiant / n).  Out of
-// line: the solve reaches it only for such vectors, and keeping its code
-// out of the solve's loop keeps that loop compact in the instruction cache.
+// components that are tiny (<= rdwarf) or huge (>= rgiant / n)
 __device__ __noinline__ double enorm_scaled(double x0, double x1, double x2, int n) {
   const double rdwarf = 3.834e-20, rgiant = 1.304e19;
   const double agiant = rgiant / double(n);
@@ -203,23 +223,49 @@ __device__ __noinline__ double enorm_scaled(double x0, double x1, double x2, int
   return sqrt(x3max * ((s2 / x3max) + (x3max * s3)));
 }
 
+constexpr double RDWARF = 3.834e-20, RGIANT = 1.304e19;
+
+// How far a norm's components are from the intermediate magnitudes (RDWARF <
+// |x| < RGIANT / 3): the largest (high word without its sign, times two) -
+// MID_LO met so far, below MID_RANGE when every component was one.  Zeros,
+// infinities and NaN are outside as well.
+constexpr unsigned MID_LO = 2u * (unsigned)((__builtin_bit_cast(unsigned long long, RDWARF) >> 32) + 1);
+constexpr unsigned MID_RANGE =
+    2u * (unsigned)(__builtin_bit_cast(unsigned long long, RGIANT / 3.0) >> 32) - MID_LO;
+__device__ __forceinline__ unsigned mid_word(double x) {
+  return ((unsigned)__double2hiint(x) << 1) - MID_LO;
+}
+
+// x x as a number of its own, never inside a fused sum
+__device__ __forceinline__ double sqr(double x) {
+#pragma clang fp contract(off)
+  return x * x;
+}
+
+__device__ __forceinline__ double fma2(double a, double b, double c, double d, double e) {
+  return __builtin_fma(a, b, __builtin_fma(c, d, e));
+}
+
 // enorm.  When every component is zero or of intermediate magnitude
 // (rdwarf < |x| < rgiant / N) MINPACK's sums reduce to s1 = s3 = x3max = 0
-// and the result to sqrt(s2), s2 the plain sum of squares in index order;
-// that case is computed here, the others by enorm_scaled.
-template <int N>
-__device__ __forceinline__ double enorm(const double* x) {
-  const double rdwarf = 3.834e-20, rgiant = 1.304e19;
-  const double agiant = rgiant / double(N);
-  // non-short-circuit operators: the test is a few compares, not a branch
-  // per component
+// and the result to sqrt(s2), s2 the plain sum of squares.  FAST: only that,
+// noting in `far` whether it was right; else the others go to enorm_scaled.
+// The sum's roundings are fixed: component R is squared first.
+template <bool FAST, int N, int R = 1>
+__device__ __forceinline__ double enorm(const double* x, unsigned& far) {
+  double sq = __builtin_fma(x[1 - R], x[1 - R], sqr(x[R]));
+  if (N > 2) sq = __builtin_fma(x[2], x[2], sq);
+  if (FAST) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) far = max(far, mid_word(x[i]));
+    return sqrt(sq);
+  }
+  const double agiant = RGIANT / double(N);
   bool mid = true;
-  double sq = 0.0;
 #pragma unroll
   for (int i = 0; i < N; ++i) {
     const double xabs = fabs(x[i]);
-    mid = mid & ((xabs == 0.0) | ((xabs > rdwarf) & (xabs < agiant)));
-    sq += xabs * xabs;
+    mid = mid & ((xabs == 0.0) | ((xabs > RDWARF) & (xabs < agiant)));
   }
   if (mid) return sqrt(sq);
   return enorm_scaled(x[0], x[1], N > 2 ? x[2] : 0.0, N);
@@ -229,10 +275,11 @@ constexpr double EPSMCH = 2.220446049250313e-16;
 constexpr double DWARF = 2.2250738585072014e-308;
 
 // qrfac with column pivoting (minpack_reduc.f90:1007-1120), m = 3, n = 2
+template <bool FAST>
 __device__ __forceinline__ void qrfac32(double a[6], int ipvt[2], double rdiag[2],
-                                        double acnorm[2], double wa[2]) {
+                                        double acnorm[2], double wa[2], unsigned& far) {
   for (int j = 0; j < 2; ++j) {
-    acnorm[j] = enorm<3>(a + 3 * j);
+    acnorm[j] = enorm<FAST, 3>(a + 3 * j, far);
     rdiag[j] = acnorm[j];
     wa[j] = rdiag[j];
     ipvt[j] = j;
@@ -245,12 +292,12 @@ __device__ __forceinline__ void qrfac32(double a[6], int ipvt[2], double rdiag[2
     ipvt[0] = 1; ipvt[1] = 0;
   }
   {
-    double ajnorm = enorm<3>(a);
+    double ajnorm = enorm<FAST, 3, 0>(a, far);
     if (ajnorm != 0.0) {
       if (a[0] < 0.0) ajnorm = -ajnorm;
       for (int i = 0; i < 3; ++i) a[i] = a[i] / ajnorm;
       a[0] = a[0] + 1.0;
-      double sum = a[0] * a[3] + a[1] * a[4] + a[2] * a[5];
+      double sum = fma2(a[2], a[5], a[1], a[4], a[0] * a[3]);
       double temp = sum / a[0];
       for (int i = 0; i < 3; ++i) a[3 + i] = a[3 + i] - temp * a[i];
       if (rdiag[1] != 0.0) {
@@ -259,7 +306,7 @@ __device__ __forceinline__ void qrfac32(double a[6], int ipvt[2], double rdiag[2
         rdiag[1] = rdiag[1] * sqrt(t2 > 0.0 ? t2 : 0.0);
         double t3 = rdiag[1] / wa[1];
         if (0.05 * (t3 * t3) <= EPSMCH) {
-          rdiag[1] = enorm<2>(a + 4);
+          rdiag[1] = enorm<FAST, 2, 0>(a + 4, far);
           wa[1] = rdiag[1];
         }
       }
@@ -268,7 +315,7 @@ __device__ __forceinline__ void qrfac32(double a[6], int ipvt[2], double rdiag[2
   }
   // j = 1 (no pivot candidates left)
   {
-    double ajnorm = enorm<2>(a + 4);
+    double ajnorm = enorm<FAST, 2, 0>(a + 4, far);
     if (ajnorm != 0.0) {
       if (a[4] < 0.0) ajnorm = -ajnorm;
       a[4] = a[4] / ajnorm;
@@ -306,13 +353,14 @@ __device__ __forceinline__ void qrsolv2(double r[6], const int ipvt[2], const do
             sn = 0.5 / sqrt(0.25 + 0.25 * (ct * ct));
             cs = sn * ct;
           }
-          r[k * 4] = cs * rkk + sn * sdiag[k];
-          double temp = cs * wa[k] + sn * qtbpj;
-          qtbpj = -(sn * wa[k]) + cs * qtbpj;
+          r[k * 4] = j == 0 ? __builtin_fma(sn, sdiag[k], cs * rkk)
+                            : __builtin_fma(cs, rkk, sn * sdiag[k]);
+          double temp = __builtin_fma(cs, wa[k], sn * qtbpj);
+          qtbpj = __builtin_fma(-sn, wa[k], cs * qtbpj);
           wa[k] = temp;
           if (k == 0) {   // i = 1: r(1,0)
-            temp = cs * r[1] + sn * sdiag[1];
-            sdiag[1] = -(sn * r[1]) + cs * sdiag[1];
+            temp = __builtin_fma(cs, r[1], sn * sdiag[1]);
+            sdiag[1] = __builtin_fma(-sn, r[1], cs * sdiag[1]);
             r[1] = temp;
           }
         }
@@ -336,9 +384,10 @@ __device__ __forceinline__ void qrsolv2(double r[6], const int ipvt[2], const do
 }
 
 // lmpar (minpack_reduc.f90:798-987), n = 2
+template <bool FAST>
 __device__ __forceinline__ void lmpar2(double r[6], const int ipvt[2], const double diag[2],
                                        const double qtb[2], double delta, double& par,
-                                       double x[2], double sdiag[2]) {
+                                       double x[2], double sdiag[2], unsigned& far) {
   const double p1 = 0.1, p001 = 1.0e-3;
   double wa1[2], wa2[2];
   int nsing = 2;
@@ -352,20 +401,20 @@ __device__ __forceinline__ void lmpar2(double r[6], const int ipvt[2], const dou
   x[0] = ipvt[0] ? wa1[1] : wa1[0];   // x[ipvt[j]] = wa1[j]
   x[1] = ipvt[0] ? wa1[0] : wa1[1];
   wa2[0] = diag[0] * x[0]; wa2[1] = diag[1] * x[1];
-  double dxnorm = enorm<2>(wa2);
+  double dxnorm = enorm<FAST, 2>(wa2, far);
   double fp = dxnorm - delta;
   if (fp <= p1 * delta) { par = 0.0; return; }
   double parl = 0.0;
   if (nsing >= 2) {
-    for (int j = 0; j < 2; ++j) wa1[j] = pick(diag, ipvt[j]) * (pick(wa2, ipvt[j]) / dxnorm);
+    wa1[0] = pick(diag, ipvt[0]) * (pick(wa2, ipvt[0]) / dxnorm);
     wa1[0] = wa1[0] / r[0];
-    wa1[1] = (wa1[1] - r[3] * wa1[0]) / r[4];
-    double temp = enorm<2>(wa1);
+    wa1[1] = __builtin_fma(pick(diag, ipvt[1]), pick(wa2, ipvt[1]) / dxnorm, -(r[3] * wa1[0])) / r[4];
+    double temp = enorm<FAST, 2>(wa1, far);
     parl = ((fp / delta) / temp) / temp;
   }
   wa1[0] = (r[0] * qtb[0]) / pick(diag, ipvt[0]);
-  wa1[1] = (r[3] * qtb[0] + r[4] * qtb[1]) / pick(diag, ipvt[1]);
-  double gnorm = enorm<2>(wa1);
+  wa1[1] = __builtin_fma(r[3], qtb[0], r[4] * qtb[1]) / pick(diag, ipvt[1]);
+  double gnorm = enorm<FAST, 2>(wa1, far);
   double paru = gnorm / delta;
   if (paru == 0.0) paru = DWARF / fmin(delta, p1);
   par = fmax(par, parl);
@@ -377,15 +426,15 @@ __device__ __forceinline__ void lmpar2(double r[6], const int ipvt[2], const dou
     wa1[0] = temp * diag[0]; wa1[1] = temp * diag[1];
     qrsolv2(r, ipvt, wa1, qtb, x, sdiag);
     wa2[0] = diag[0] * x[0]; wa2[1] = diag[1] * x[1];
-    dxnorm = enorm<2>(wa2);
+    dxnorm = enorm<FAST, 2>(wa2, far);
     temp = fp;
     fp = dxnorm - delta;
     if (fabs(fp) <= p1 * delta || (parl == 0.0 && fp <= temp && temp < 0.0) || iter == 10) break;
-    for (int j = 0; j < 2; ++j) wa1[j] = pick(diag, ipvt[j]) * (pick(wa2, ipvt[j]) / dxnorm);
+    wa1[0] = pick(diag, ipvt[0]) * (pick(wa2, ipvt[0]) / dxnorm);
     wa1[0] = wa1[0] / sdiag[0];
-    wa1[1] = wa1[1] - r[1] * wa1[0];
+    wa1[1] = __builtin_fma(pick(diag, ipvt[1]), pick(wa2, ipvt[1]) / dxnorm, -(r[1] * wa1[0]));
     wa1[1] = wa1[1] / sdiag[1];
-    temp = enorm<2>(wa1);
+    temp = enorm<FAST, 2>(wa1, far);
     double parc = ((fp / delta) / temp) / temp;
     if (fp > 0.0) parl = fmax(parl, par);
     if (fp < 0.0) paru = fmin(paru, par);
@@ -393,119 +442,183 @@ __device__ __forceinline__ void lmpar2(double r[6], const int ipvt[2], const dou
   }
 }
 
+// Where a solve stands between two evaluations (lmder's variables that it
+// still needs): the point, R and Q^T f of the factored Jacobian there and the
+// step bound.
+struct LmState {
+  double x[2], r[3], qtf[2], diag[2];   // r: r(0,0), r(0,1), r(1,1)
+  double delta, par, xnorm, fnorm, gnorm;
+  int swapped;                          // columns pivoted
+  int iter, nfev, info;
+};
+
+// Jacobian at the point of s, its factorisation, Q^T fvec and the gradient
+template <bool FAST>
+__device__ __forceinline__ void lm_factor(const ContactPair& cp, const Jet& s,
+                                          const double fvec[3], bool first, LmState& t,
+                                          unsigned& far) {
+  double fjac[6], wa1[2], wa2[2], wa3[2], wa4[3];
+  int ipvt[2];
+  fcn_j(cp, s, fjac);
+  qrfac32<FAST>(fjac, ipvt, wa1, wa2, wa3, far);
+  t.swapped = ipvt[0];
+  if (first) {
+    for (int j = 0; j < 2; ++j) t.diag[j] = (wa2[j] == 0.0) ? 1.0 : wa2[j];
+    wa3[0] = t.diag[0] * t.x[0]; wa3[1] = t.diag[1] * t.x[1];
+    t.xnorm = enorm<FAST, 2>(wa3, far);
+    t.delta = 100.0 * t.xnorm;
+    if (t.delta == 0.0) t.delta = 100.0;
+  }
+  wa4[0] = fvec[0]; wa4[1] = fvec[1]; wa4[2] = fvec[2];
+  if (fjac[0] != 0.0) {
+    double sum = fma2(fjac[2], wa4[2], fjac[1], wa4[1], fjac[0] * wa4[0]);
+    double temp = -sum / fjac[0];
+    for (int i = 0; i < 3; ++i) wa4[i] += fjac[i] * temp;
+  }
+  t.r[0] = wa1[0];
+  t.r[1] = fjac[3];
+  t.qtf[0] = wa4[0];
+  if (fjac[4] != 0.0) {
+    double sum = __builtin_fma(fjac[5], wa4[2], fjac[4] * wa4[1]);
+    double temp = -sum / fjac[4];
+    wa4[1] += fjac[4] * temp;
+    wa4[2] += fjac[5] * temp;
+  }
+  t.r[2] = wa1[1];
+  t.qtf[1] = wa4[1];
+  double gnorm = 0.0;
+  if (t.fnorm != 0.0) {
+    for (int j = 0; j < 2; ++j) {
+      const double wl = pick(wa2, ipvt[j]);
+      if (wl != 0.0) {
+        double sum = (j == 0) ? t.r[0] * (t.qtf[0] / t.fnorm)
+                              : __builtin_fma(t.r[1], t.qtf[0] / t.fnorm,
+                                              t.r[2] * (t.qtf[1] / t.fnorm));
+        gnorm = fmax(gnorm, fabs(sum / wl));
+      }
+    }
+  }
+  t.gnorm = gnorm;
+  if (gnorm <= 0.0) { t.info = 4; return; }   // gtol = 0
+  t.diag[0] = fmax(t.diag[0], wa2[0]);
+  t.diag[1] = fmax(t.diag[1], wa2[1]);
+}
+
 // lmder with lmder1's settings (minpack_reduc.f90:243-640, :732-745):
-// mode 1, factor 100, maxfev 300, ftol = xtol = sqrt(eps), gtol = 0.
-// Returns the number of function evaluations; *info_out = MINPACK's info
-// (1 converged, 4 zero gradient, 5 maxfev, 6 tolerances too small for a
-// further reduction: MINPACK's 6-8); cur = the Jet of the returned x.
-// maxfev below 300 only for a network-seeded first attempt.
-__device__ int lm_solve(const ContactPair& cp, double x[2], int* info_out, Jet& cur,
-                        int maxfev = 300) {
+// mode 1, factor 100, maxfev 300, ftol = xtol = sqrt(eps), gtol = 0, from
+// the state s (nfev = 0: from its x) until info is set: MINPACK's info (1
+// converged, 4 zero gradient, 5 maxfev, 6 tolerances too small for a further
+// reduction: MINPACK's 6-8).  FAST: up to the first evaluation whose norms
+// need MINPACK's scaled sums, which is not taken (false returned, s before
+// it).
+template <bool FAST>
+__device__ __forceinline__ bool lm_run(const ContactPair& cp, LmState& s, int maxfev) {
   const double tol = 1.4901161193847656e-08;
   const double p1 = 0.1, p5 = 0.5, p25 = 0.25, p75 = 0.75, p0001 = 1.0e-4;
-  double fvec[3], fjac[6], diag[2], qtf[2], wa1[2], wa2[2], wa3[2], wa4[3];
-  int ipvt[2];
-  int info = 0, nfev = 1, iter = 1;
-  double delta = 0.0, xnorm = 0.0, par = 0.0;
-  Jet trial;
-  support(cp, x, cur, fvec);
-  double fnorm = enorm<3>(fvec);
   for (;;) {
-    fcn_j(cp, cur, fjac);
-    qrfac32(fjac, ipvt, wa1, wa2, wa3);
-    if (iter == 1) {
-      for (int j = 0; j < 2; ++j) diag[j] = (wa2[j] == 0.0) ? 1.0 : wa2[j];
-      wa3[0] = diag[0] * x[0]; wa3[1] = diag[1] * x[1];
-      xnorm = enorm<2>(wa3);
-      delta = 100.0 * xnorm;
-      if (delta == 0.0) delta = 100.0;
-    }
-    wa4[0] = fvec[0]; wa4[1] = fvec[1]; wa4[2] = fvec[2];
-    // Q^T fvec
-    if (fjac[0] != 0.0) {
-      double sum = fjac[0] * wa4[0] + fjac[1] * wa4[1] + fjac[2] * wa4[2];
-      double temp = -sum / fjac[0];
-      for (int i = 0; i < 3; ++i) wa4[i] += fjac[i] * temp;
-    }
-    fjac[0] = wa1[0];
-    qtf[0] = wa4[0];
-    if (fjac[4] != 0.0) {
-      double sum = fjac[4] * wa4[1] + fjac[5] * wa4[2];
-      double temp = -sum / fjac[4];
-      wa4[1] += fjac[4] * temp;
-      wa4[2] += fjac[5] * temp;
-    }
-    fjac[4] = wa1[1];
-    qtf[1] = wa4[1];
-    double gnorm = 0.0;
-    if (fnorm != 0.0) {
-      for (int j = 0; j < 2; ++j) {
-        const double wl = pick(wa2, ipvt[j]);
-        if (wl != 0.0) {
-          double sum = (j == 0) ? fjac[0] * (qtf[0] / fnorm)
-                                : fjac[3] * (qtf[0] / fnorm) + fjac[4] * (qtf[1] / fnorm);
-          gnorm = fmax(gnorm, fabs(sum / wl));
-        }
-      }
-    }
-    if (gnorm <= 0.0) { info = 4; break; }   // gtol = 0
-    diag[0] = fmax(diag[0], wa2[0]);
-    diag[1] = fmax(diag[1], wa2[1]);
-    for (;;) {
-      lmpar2(fjac, ipvt, diag, qtf, delta, par, wa1, wa2);
+    LmState t = s;
+    unsigned far = 0;
+    const bool first = s.nfev == 0;
+    const int ipvt[2] = {t.swapped, 1 - t.swapped};
+    double fjac[6] = {t.r[0], 0.0, 0.0, t.r[1], t.r[2], 0.0};
+    double wa1[2] = {0.0, 0.0}, wa2[2] = {t.x[0], t.x[1]}, wa3[2], wa4[3], pnorm = 0.0;
+    if (!first) {
+      lmpar2<FAST>(fjac, ipvt, t.diag, t.qtf, t.delta, t.par, wa1, wa2, far);
       wa1[0] = -wa1[0]; wa1[1] = -wa1[1];
-      wa2[0] = x[0] + wa1[0]; wa2[1] = x[1] + wa1[1];
-      wa3[0] = diag[0] * wa1[0]; wa3[1] = diag[1] * wa1[1];
-      double pnorm = enorm<2>(wa3);
-      if (iter == 1) delta = fmin(delta, pnorm);
-      support(cp, wa2, trial, wa4);
-      nfev++;
-      double fnorm1 = enorm<3>(wa4);
+      wa2[0] = t.x[0] + wa1[0]; wa2[1] = t.x[1] + wa1[1];
+      wa3[0] = t.diag[0] * wa1[0]; wa3[1] = t.diag[1] * wa1[1];
+      pnorm = enorm<FAST, 2, 0>(wa3, far);
+      if (t.iter == 1) t.delta = fmin(t.delta, pnorm);
+    }
+    Jet trial;
+    support(cp, wa2, trial, wa4);
+    t.nfev++;
+    const double fnorm1 = enorm<FAST, 3>(wa4, far);
+    bool accept = true;
+    if (first) {
+      t.fnorm = fnorm1;
+    } else {
       double actred = -1.0;
-      if (p1 * fnorm1 < fnorm) { double t = fnorm1 / fnorm; actred = 1.0 - t * t; }
+      if (p1 * fnorm1 < t.fnorm) { double q = fnorm1 / t.fnorm; actred = 1.0 - q * q; }
       {
         double t0 = pick(wa1, ipvt[0]), t1 = pick(wa1, ipvt[1]);
-        wa3[0] = fjac[0] * t0 + fjac[3] * t1;
-        wa3[1] = fjac[4] * t1;
+        wa3[0] = __builtin_fma(t.r[1], t1, t.r[0] * t0);
+        wa3[1] = t.r[2] * t1;
       }
-      double temp1 = enorm<2>(wa3) / fnorm;
-      double temp2 = (sqrt(par) * pnorm) / fnorm;
-      double prered = temp1 * temp1 + (temp2 * temp2) / p5;
-      double dirder = -(temp1 * temp1 + temp2 * temp2);
+      double temp1 = enorm<FAST, 2, 0>(wa3, far) / t.fnorm;
+      double temp2 = (sqrt(t.par) * pnorm) / t.fnorm;
+      const double q1 = sqr(temp1), q2 = sqr(temp2);
+      double prered = q1 + q2 / p5;
+      double dirder = -(q1 + q2);
       double ratio = 0.0;
       if (prered != 0.0) ratio = actred / prered;
       if (ratio <= p25) {
         double temp = (actred >= 0.0) ? p5 : p5 * dirder / (dirder + p5 * actred);
-        if (p1 * fnorm1 >= fnorm || temp < p1) temp = p1;
-        delta = temp * fmin(delta, pnorm / p1);
-        par = par / temp;
-      } else if (par == 0.0 || ratio >= p75) {
-        delta = pnorm / p5;
-        par = p5 * par;
+        if (p1 * fnorm1 >= t.fnorm || temp < p1) temp = p1;
+        t.delta = temp * fmin(t.delta, pnorm / p1);
+        t.par = t.par / temp;
+      } else if (t.par == 0.0 || ratio >= p75) {
+        t.delta = pnorm / p5;
+        t.par = p5 * t.par;
       }
-      if (ratio >= p0001) {
-        x[0] = wa2[0]; x[1] = wa2[1];
-        wa2[0] = diag[0] * x[0]; wa2[1] = diag[1] * x[1];
-        fvec[0] = wa4[0]; fvec[1] = wa4[1]; fvec[2] = wa4[2];
-        cur = trial;
-        xnorm = enorm<2>(wa2);
-        fnorm = fnorm1;
-        iter++;
+      accept = ratio >= p0001;
+      if (accept) {
+        t.x[0] = wa2[0]; t.x[1] = wa2[1];
+        wa2[0] = t.diag[0] * t.x[0]; wa2[1] = t.diag[1] * t.x[1];
+        t.xnorm = enorm<FAST, 2, 0>(wa2, far);
+        t.fnorm = fnorm1;
+        t.iter++;
       }
       bool small = fabs(actred) <= tol && prered <= tol && p5 * ratio <= 1.0;
-      if (small || delta <= tol * xnorm) { info = 1; break; }
-      if (nfev >= maxfev) { info = 5; break; }
-      if ((fabs(actred) <= EPSMCH && prered <= EPSMCH && p5 * ratio <= 1.0) ||
-          delta <= EPSMCH * xnorm || gnorm <= EPSMCH) {
-        info = 6;
-        break;
+      if (small || t.delta <= tol * t.xnorm) {
+        t.info = 1;
+      } else if (t.nfev >= maxfev) {
+        t.info = 5;
+      } else if ((fabs(actred) <= EPSMCH && prered <= EPSMCH && p5 * ratio <= 1.0) ||
+                 t.delta <= EPSMCH * t.xnorm || t.gnorm <= EPSMCH) {
+        t.info = 6;
       }
-      if (ratio >= p0001) break;
     }
-    if (info != 0) break;
+    if (t.info == 0 && accept) lm_factor<FAST>(cp, trial, wa4, first, t, far);
+    if (FAST && far >= MID_RANGE) return false;
+    s = t;
+    if (s.info != 0) return true;
   }
-  *info_out = info;
-  return nfev;
+}
+__device__ __noinline__ void lm_rest(const ContactPair* cp, LmState* s, int maxfev) {
+  const ContactPair c = *cp;
+  LmState t = *s;
+  lm_run<false>(c, t, maxfev);
+  *s = t;
+}
+
+// The solve from x.  Returns the number of function evaluations; *info_out =
+// MINPACK's info; cur = the Jet of the returned x (evaluated once more: kept
+// through the loop beside the trial point's it costs 36 registers).  maxfev
+// below 300 only for a network-seeded first attempt.
+// The solve is a serial chain of some 2000 instructions an evaluation.  Its
+// 13 norms each had a branch to the scaled sums, a call in the loop, for
+// components that hardly ever come (41 norms of 1e7 evaluations in a dense
+// suspension): the loop now runs without them, and a solve that meets one
+// goes on from there out of line.  Launches of 16 to 5e5 solves: 70 -> 64 us
+// (1e4 particles on 64^3), 200 -> 177 (123457, four points), 369 -> 326 (1e6
+// mixed), 2840 -> 2290 (2e6 in 5 % by volume).
+__device__ int lm_solve(const ContactPair& cp, double x[2], int* info_out, Jet& cur,
+                        int maxfev = 300) {
+  LmState s{};
+  s.x[0] = x[0]; s.x[1] = x[1];
+  s.iter = 1;
+  if (!lm_run<true>(cp, s, maxfev)) {
+    ContactPair c = cp;   // copies: these two live in memory, those of the loop do not
+    LmState t = s;
+    lm_rest(&c, &t, maxfev);
+    s = t;
+  }
+  x[0] = s.x[0]; x[1] = s.x[1];
+  double f[3];
+  support(cp, x, cur, f);
+  *info_out = s.info;
+  return s.nfev;
 }
 
 struct ContactOut {
