@@ -30,12 +30,6 @@ __device__ __forceinline__ Sym3 ell_matrix(const double q[4], double a, double b
   return e;
 }
 
-__device__ __forceinline__ void symv(const Sym3& e, const double v[3], double o[3]) {
-  o[0] = e.xx * v[0] + e.xy * v[1] + e.xz * v[2];
-  o[1] = e.xy * v[0] + e.yy * v[1] + e.yz * v[2];
-  o[2] = e.xz * v[0] + e.yz * v[1] + e.zz * v[2];
-}
-
 // Perram-Wertheim separation test.  For ellipsoids x^T E^-1 x <= 1 about
 // centres b1, b2 and r = b2 - b1,
 //   F(l) = l (1 - l) r^T [(1 - l) E1 + l E2]^-1 r,   0 < l < 1,
