@@ -477,7 +477,8 @@ int gp_field_file_read(const char *path, int n, double *f);
  * from the reference's RAN1 / GAUSS sequence, initial amplitudes 0 as
  * INITIATION_FORCING_NEW sets them for INIT_FLUID_VELOCITY <= 2) and
  * CHECK_CFL (check_cfl.f90:61-110).  Velocity and spectral state stay in
- * device memory (rocFFT, double precision); gp_dns_bind hands velocity and
+ * device memory (double precision; transforms of gp_fft.h, or rocFFT for
+ * lengths without a plan there); gp_dns_bind hands velocity and
  * a spectrally computed vorticity to a particle context without a host
  * copy.  Grids: n^3 points, the transform grid x = (i-1) L / n; arrays
  * double[3][n][n][n], x fastest.                                         */
