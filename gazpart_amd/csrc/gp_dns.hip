@@ -648,27 +648,28 @@ __global__ __launch_bounds__((RowX<N, 1>::threads)) void k_fx_cross(const double
     }
     if (threadIdx.x == 0) part[blockIdx.x] = red[0];
   } else {
-    double t0[3][E];
+    // A pair of lines is always two rows of one quantity: the rounding of a
+    // transform goes by the larger of its two parts, and velocity and
+    // vorticity differ by the wavenumber, that is, by the unit of length
+    double2 p[3][E];
 #pragma unroll
-    for (int half = 0; half < 2; ++half) {
+    for (int c = 0; c < 3; ++c) {
+      load_pair<N, 1>(B + c * g.nc, B + c * g.nc + g.pitch, r0, ro.on, ro.t, p[c]);
+      gpfft::fft<N, 1, 1, 1>(&p[c], x, tw, ro.t);
+      __builtin_amdgcn_sched_barrier(0);
+    }
 #pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        const long long r = c * g.nc + half * g.pitch;
-        load_pair<N, 1>(B + r, A + r, r0, ro.on, ro.t, v[c]);   // velocity and vorticity
-        gpfft::fft<N, 1, 1, 1>(&v[c], x, tw, ro.t);
-        __builtin_amdgcn_sched_barrier(0);
-      }
+    for (int c = 0; c < 3; ++c) {
+      load_pair<N, 1>(A + c * g.nc, A + c * g.nc + g.pitch, r0, ro.on, ro.t, v[c]);
+      gpfft::fft<N, 1, 1, 1>(&v[c], x, tw, ro.t);
+      __builtin_amdgcn_sched_barrier(0);
+    }
 #pragma unroll
-      for (int m = 0; m < E; ++m) {
-        const double2 p = v[0][m], q = v[1][m], r = v[2][m];
-        const double c0 = q.x * r.y - r.x * q.y, c1 = r.x * p.y - p.x * r.y,
-                     c2 = p.x * q.y - q.x * p.y;
-        if (half == 0) {
-          t0[0][m] = c0; t0[1][m] = c1; t0[2][m] = c2;
-        } else {
-          v[0][m] = {t0[0][m], c0}; v[1][m] = {t0[1][m], c1}; v[2][m] = {t0[2][m], c2};
-        }
-      }
+    for (int m = 0; m < E; ++m) {
+      const double2 zx = v[0][m], zy = v[1][m], zz = v[2][m];
+      v[0][m] = {p[1][m].x * zz.x - p[2][m].x * zy.x, p[1][m].y * zz.y - p[2][m].y * zy.y};
+      v[1][m] = {p[2][m].x * zx.x - p[0][m].x * zz.x, p[2][m].y * zx.y - p[0][m].y * zz.y};
+      v[2][m] = {p[0][m].x * zy.x - p[1][m].x * zx.x, p[0][m].y * zy.y - p[1][m].y * zx.y};
     }
   }
 #pragma unroll

@@ -374,3 +374,26 @@ def test_gpu_lengths_match_oracle(n, reuse):
     assert np.abs(w - wr).max() <= 1e-11 * np.abs(wr).max()
     assert abs(d.info()["eps"] - s.eps) <= 1e-11 * s.eps
     assert not np.array_equal(u, u0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [36, 48, 64, 100])
+@pytest.mark.parametrize("exp2", [-20, 20])
+def test_gpu_unit_of_length_changes_nothing(n, exp2):
+    """The same flow in another unit of length: velocity, viscosity and length
+    times powers of two.  Velocity and vorticity are then 2^20 times further
+    apart or closer, which no transform may mix.  1e-13 of the largest
+    magnitude: three steps of seven transforms, each 1e-16 log2(n^3) <= 2e-15
+    at random (4e-14 if all of them added up)."""
+    from gazpart_amd.dns import Dns
+    u0 = random_velocity(n, 4.0, 70 + n)
+    nu, dt, ns = 0.01, 0.2 / n, 3
+    out = []
+    for s in (1.0, 2.0 ** exp2):
+        d = Dns(n, L2PI * s, nu * s * s, dt)
+        d.set_velocity(u0 * s)
+        d.step(ns)
+        out.append((d.velocity() / s, d.vorticity()))
+    for a, b in zip(*out):
+        assert np.abs(a - b).max() <= 1e-13 * np.abs(a).max()
+    assert not np.array_equal(out[0][0], u0)
