@@ -1,0 +1,105 @@
+"""Parts of the device headers compiled for the CPU: what no result shows
+(which of two ways a solve takes, an error in the middle of a transfer) is
+looked at there.  A header of a few lines stands in for HIP's."""
+import os
+import subprocess
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "gazpart_amd",
+                    "csrc")
+
+HIP_STUB = r"""
+#pragma once
+#include <algorithm>
+#include <cmath>
+#include <cstring>
+using std::max; using std::min;
+#define __device__
+#define __host__
+#define __forceinline__ inline
+#define __noinline__ __attribute__((noinline))
+inline int __double2hiint(double x) {
+  unsigned long long u;
+  std::memcpy(&u, &x, 8);
+  return (int)(u >> 32);
+}
+"""
+
+
+def run(tmp_path, stub, src, *flags):
+    (tmp_path / "hip").mkdir()
+    (tmp_path / "hip" / "hip_runtime.h").write_text(stub)
+    (tmp_path / "t.cpp").write_text(src)
+    exe = str(tmp_path / "t")
+    subprocess.run(["g++", "-O2", "-std=c++17", "-pthread", f"-I{tmp_path}", f"-I{CSRC}", *flags,
+                    str(tmp_path / "t.cpp"), "-o", exe], check=True)
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, (r.returncode, r.stdout, r.stderr)
+    return r.stdout
+
+
+CONTACT = r"""
+#include <cstdio>
+#include <random>
+#include "gp_contact.h"
+using namespace gp;
+int main() {
+  std::mt19937_64 g(5);
+  std::normal_distribution<double> nd;
+  std::uniform_real_distribution<double> un(0, 1);
+  // spheres; spheroids with the x axis, and with any common axis; spheroids;
+  // tri-axial bodies; a sphere and a spheroid
+  for (int kind = 0; kind < 6; ++kind) {
+    const int n = 4000;
+    int left = 0, differ = 0;
+    for (int k = 0; k < n; ++k) {
+      const double a = 0.02;
+      double b = kind == 0 || kind == 5 ? a : a / (1 + 2 * un(g)), c = b;
+      if (kind == 4) c = a / (1 + 2 * un(g));
+      const double b2 = kind == 5 ? a / 2 : b, c2 = kind == 5 ? a / 2 : c;
+      double q1[4] = {1, 0, 0, 0}, q2[4] = {1, 0, 0, 0}, d[3], bi[3], bj[3], r = 0;
+      auto turn = [&](double* q) {
+        double s = 0;
+        for (int i = 0; i < 4; ++i) { q[i] = nd(g); s += q[i] * q[i]; }
+        for (int i = 0; i < 4; ++i) q[i] /= std::sqrt(s);
+      };
+      if (kind != 1) { turn(q1); turn(q2); }
+      if (kind == 2) std::copy(q1, q1 + 4, q2);
+      for (double& x : d) { x = nd(g); r += x * x; }
+      r = (0.5 + 0.6 * un(g)) * 2 * a / std::sqrt(r);
+      ContactPair cp;
+      for (int i = 0; i < 3; ++i) {
+        cp.b1[i] = 1 + un(g);
+        cp.b2[i] = cp.b1[i] + r * d[i];
+      }
+      cp.E1 = ell_matrix(q1, a, b, c);
+      cp.E2 = ell_matrix(q2, a, b2, c2);
+      double e[3], s = 0;   // the start on the line of centres
+      for (int i = 0; i < 3; ++i) { e[i] = cp.b1[i] - cp.b2[i]; s += e[i] * e[i]; }
+      LmState t{};
+      t.x[1] = std::asin(e[2] / std::sqrt(s));
+      t.x[0] = std::acos(std::min(1.0, std::max(-1.0, e[0] / std::sqrt(s) / std::cos(t.x[1]))));
+      t.iter = 1;
+      LmState f = t;
+      lm_rest(&cp, &f, 300);
+      if (!lm_run<true>(cp, t, 300)) {
+        ++left;
+        lm_rest(&cp, &t, 300);
+      }
+      differ += t.nfev != f.nfev || t.info != f.info || t.x[0] != f.x[0] || t.x[1] != f.x[1];
+    }
+    std::printf("%d %d\n", left, differ);
+  }
+}
+"""
+
+
+def test_contact_solves_stay_in_the_plain_loop(tmp_path):
+    """Bodies of any symmetry solve in the loop without scaled sums (an exact
+    zero or its residue in a component leaves the norm as it is), with the
+    iterates of the run that has them.  A solve may leave where every
+    component is tiny: at most 1 in 1000."""
+    out = run(tmp_path, HIP_STUB, CONTACT, "-ffp-contract=off")
+    for left, differ in (map(int, line.split()) for line in out.splitlines()):
+        assert left <= 4 and differ == 0, out
