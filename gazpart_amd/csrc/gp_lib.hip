@@ -1857,8 +1857,11 @@ __global__ __launch_bounds__(GREEDY_BLOCK) void k_greedy_rounds(
 }
 
 // every round in one workgroup, one launch instead of four, where the last
-// known count of solves (which bounds the contacts and, unlike them, does not
-// depend on the velocities) is at most GREEDY_FEW; any number is right.
+// count of the present particles' solves (which bounds the contacts and,
+// unlike them, does not depend on the velocities) is at most GREEDY_FEW; any
+// number is right, but 1.6e5 contacts take 6.5 ms instead of 4.3.  A new set of
+// particles starts unknown, and a captured graph goes when a count read back
+// is larger.
 // Bound by the launches: 1e4 particles on 64^3 (some ten contacts) 13.7 us in
 // four launches, 5.0 us in one (a pass of 64 steps 13.2 -> 12.1 ms).
 // Thousands of contacts want more than one workgroup.
@@ -2333,7 +2336,9 @@ struct gp_ctx {
   int ep_par = 0;
   bool ep_step = false;            // this step solves ahead
   unsigned long long last_nlm = 0; // last known count of contact solves
-  bool nlm_known = false;
+  bool solved = false;             // a pass over the present particles and species has solved
+  bool nlm_known = false;          // and last_nlm is a count of theirs
+  bool g_few = false;              // gexec has its matching rounds in one workgroup
 };
 
 // ---------------------------------------------------------------------------
@@ -2370,6 +2375,10 @@ static int scratch_init(gp_ctx* ctx) {
 static void drop_graph(gp_ctx* ctx) {
   if (ctx->gexec) hipGraphExecDestroy(ctx->gexec);
   ctx->gexec = nullptr;
+}
+
+static bool greedy_few(const gp_ctx* ctx) {
+  return ctx->nlm_known && ctx->last_nlm <= GREEDY_FEW;
 }
 
 // bf16 block offsets (in shorts) and bias offsets of the seed network
@@ -3042,6 +3051,7 @@ int gp_set_species(gp_ctx* ctx, int nspec, const double* rows) {
   }
   hipStreamSynchronize(ctx->st);
   drop_graph(ctx);
+  ctx->solved = ctx->nlm_known = false;
   std::vector<Species> h((size_t)nspec);
   double emax = 0.0;
   for (int s = 0; s < nspec; ++s) {
@@ -3186,6 +3196,7 @@ int gp_set_particles(gp_ctx* ctx, int np, const double* state, const int* specie
   hipStreamSynchronize(ctx->st2);
   hipStreamSynchronize(ctx->st3);
   drop_graph(ctx);
+  ctx->solved = ctx->nlm_known = false;
   ctx->contacts_valid = false;
   ctx->lists_sized = false;
   ctx->pipe_prev = false;
@@ -3880,7 +3891,8 @@ static int launch_contacts_solve(gp_ctx* ctx) {
                        c + 4, c + 7, ctx->d_err);
   }
   mark(ctx, 3);
-  if (ctx->nlm_known && ctx->last_nlm <= GREEDY_FEW) {
+  ctx->solved = true;
+  if (greedy_few(ctx)) {
     hipLaunchKernelGGL(k_greedy_few, dim3(1), dim3(GREEDY_BLOCK), 0, ctx->st, ctx->act, c + 2,
                        ctx->act_cap, ctx->mark, ctx->used, ctx->act_status, c + 6);
   } else {
@@ -4086,6 +4098,7 @@ static int capture_graph(gp_ctx* ctx) {
   ctx->g_cur = ctx->cur;
   ctx->g_perm = ctx->perm;
   ctx->g_perm_identity = ctx->perm_identity;
+  ctx->g_few = greedy_few(ctx);
   HIPCHK(hipStreamBeginCapture(ctx->st, hipStreamCaptureModeThreadLocal));
   int rc = launch_steps<VT>(ctx, graph_unit(ctx));
   hipGraph_t g = nullptr;
@@ -4116,7 +4129,8 @@ static int capture_graph(gp_ctx* ctx) {
 // register budget; 4 queue behind them).  No effect on results.
 static void choose_lm_waves(gp_ctx* ctx, unsigned long long nlm) {
   ctx->last_nlm = nlm;
-  ctx->nlm_known = true;
+  ctx->nlm_known = ctx->solved;
+  if (ctx->gexec && ctx->g_few && !greedy_few(ctx)) drop_graph(ctx);   // the stream is idle
   if (ctx->prm.lm_waves > 0) return;
   const unsigned long long lanes = (unsigned long long)ctx->nsimd * 64ull;
   ctx->lm_waves = ctx->nsimd * (nlm >= 4 * lanes ? 4 : nlm >= lanes ? 2 : 1);
