@@ -3128,7 +3128,7 @@ static hipError_t send_state(gp_ctx* ctx, const double* state, const int* specie
   hipError_t e = ctx->xf.reserve(n, (size_t)ch * row, true);
   if (e != hipSuccess) return e;
   auto p = pstate<VT>(ctx, 0);
-  return gpx::Xfer::run(n, ((long long)np + ch - 1) / ch, [&](int b, long long q) {
+  return gpx::Xfer::run(n, ((long long)np + ch - 1) / ch, ctx->st, [&](int b, long long q) {
     gpx::Xfer& x = ctx->xf;
     hipError_t r = q >= n ? hipEventSynchronize(x.ev[b]) : hipSuccess;   // the buffer's last chunk
     if (r != hipSuccess) return r;
@@ -3164,7 +3164,7 @@ static hipError_t fetch_state(gp_ctx* ctx, double* state) {
   hipLaunchKernelGGL(k_pos_of_id<VT>, dim3(nblk(ctx->np)), dim3(BLOCK), 0, ctx->st, p,
                      ctx->pos_of_id, ctx->np);
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  return gpx::Xfer::run(n, ((long long)np + ch - 1) / ch, [&](int b, long long q) {
+  return gpx::Xfer::run(n, ((long long)np + ch - 1) / ch, ctx->st, [&](int b, long long q) {
     gpx::Xfer& x = ctx->xf;
     const size_t i0 = (size_t)q * ch, m = std::min<size_t>(ch, np - i0);
     hipLaunchKernelGGL(k_gather_chunk<VT>, dim3(nblk((long long)m)), dim3(BLOCK), 0, ctx->st, p,

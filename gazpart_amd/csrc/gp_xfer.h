@@ -19,7 +19,6 @@
 #include <atomic>
 #include <cstddef>
 #include <cstring>
-#include <system_error>
 #include <thread>
 
 namespace gpx {
@@ -73,8 +72,10 @@ struct Xfer {
   }
 
   // f(worker, chunk) for every chunk, workers in parallel (a chunk's number
-  // modulo n is its worker); the first error ends it
-  template <typename F> static hipError_t run(int n, long long chunks, F&& f) {
+  // modulo n is its worker); the first error ends it, when what was queued on
+  // the stream by then (it uses the buffers) is complete
+  template <typename F>
+  static hipError_t run(int n, long long chunks, hipStream_t st, F&& f) {
     std::atomic<int> err{(int)hipSuccess};
     int device = 0;
     (void)hipGetDevice(&device);
@@ -93,13 +94,14 @@ struct Xfer {
           (void)hipSetDevice(device);   // a thread starts on device 0
           work(b);
         });
-      } catch (const std::system_error&) {
-        break;   // no more threads to be had: their chunks are taken below
+      } catch (...) {
+        break;   // no more threads, or no memory for one: their chunks are taken below
       }
     }
     work(0);
     for (int b = started; b < n; ++b) work(b);
     for (int b = 1; b < started; ++b) th[b].join();
+    if (err.load() != (int)hipSuccess) (void)hipStreamSynchronize(st);
     return (hipError_t)err.load();
   }
 
@@ -119,7 +121,7 @@ struct Xfer {
     const size_t ch = chunk_of(bytes, n);
     hipError_t e = reserve(n, ch, false);
     if (e != hipSuccess) return e;
-    return run(n, (long long)((bytes + ch - 1) / ch), [&](int b, long long q) {
+    return run(n, (long long)((bytes + ch - 1) / ch), st, [&](int b, long long q) {
       const size_t o = (size_t)q * ch, m = std::min(ch, bytes - o);
       hipError_t r = hipMemcpyAsync(pin[b], (const char*)src + o, m, hipMemcpyDeviceToHost, st);
       if (r == hipSuccess) r = hipEventRecord(ev[b], st);
@@ -136,7 +138,7 @@ struct Xfer {
     const size_t ch = chunk_of(bytes, n);
     hipError_t e = reserve(n, ch, false);
     if (e != hipSuccess) return e;
-    e = run(n, (long long)((bytes + ch - 1) / ch), [&](int b, long long q) {
+    e = run(n, (long long)((bytes + ch - 1) / ch), st, [&](int b, long long q) {
       const size_t o = (size_t)q * ch, m = std::min(ch, bytes - o);
       // the buffer's last chunk has left it
       hipError_t r = q >= n ? hipEventSynchronize(ev[b]) : hipSuccess;

@@ -103,3 +103,80 @@ def test_contact_solves_stay_in_the_plain_loop(tmp_path):
     out = run(tmp_path, HIP_STUB, CONTACT, "-ffp-contract=off")
     for left, differ in (map(int, line.split()) for line in out.splitlines()):
         assert left <= 4 and differ == 0, out
+
+
+XFER_STUB = r"""
+#pragma once
+#include <atomic>
+#include <cstdlib>
+#include <cstring>
+typedef int hipError_t;
+typedef void* hipEvent_t;
+typedef void* hipStream_t;
+enum { hipSuccess = 0, hipErrorUnknown = 999 };
+enum { hipEventDisableTiming, hipMemcpyDeviceToHost, hipMemcpyHostToDevice };
+inline std::atomic<int> calls{0}, copies{0}, last_copy{0}, waited{0}, fail_at{-1};
+inline hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
+inline hipError_t hipSetDevice(int) { return hipSuccess; }
+inline hipError_t hipEventCreateWithFlags(hipEvent_t* e, int) { *e = e; return hipSuccess; }
+inline hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
+inline hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+inline hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+inline hipError_t hipHostMalloc(void** p, size_t n) { *p = std::malloc(n); return hipSuccess; }
+inline hipError_t hipHostFree(void* p) { std::free(p); return hipSuccess; }
+inline hipError_t hipMalloc(void** p, size_t n) { return hipHostMalloc(p, n); }
+inline hipError_t hipFree(void* p) { return hipHostFree(p); }
+inline hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, int, hipStream_t) {
+  if (copies++ == fail_at) return hipErrorUnknown;
+  std::memcpy(d, s, n);
+  last_copy = ++calls;
+  return hipSuccess;
+}
+inline hipError_t hipStreamSynchronize(hipStream_t) { waited = ++calls; return hipSuccess; }
+"""
+
+XFER = r"""
+#include <cstdio>
+#include <new>
+#include <vector>
+#include "gp_xfer.h"
+static std::atomic<int> news_left{-1};   // -1: any number
+void* operator new(size_t n) {
+  if (news_left >= 0 && news_left-- == 0) throw std::bad_alloc();
+  return std::malloc(n);
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, size_t) noexcept { std::free(p); }
+int main() {
+  const size_t n = (size_t)37 << 20;
+  std::vector<char> a(n), b(n);
+  for (size_t i = 0; i < n; ++i) a[i] = (char)(i * 7 + (i >> 12));
+  gpx::Xfer x;
+  // memory for no, one, two threads
+  for (int k = 0; k < 3; ++k) {
+    for (int way = 0; way < 2; ++way) {
+      std::fill(b.begin(), b.end(), 0);
+      news_left = k;
+      const hipError_t e = way ? x.h2d(b.data(), a.data(), n, nullptr) : x.d2h(b.data(), a.data(), n, nullptr);
+      news_left = -1;
+      if (e != hipSuccess || a != b) return 1;
+    }
+  }
+  // an error ends a transfer when the copies before it are complete
+  for (int at = 0; at < 9; at += 2) {
+    copies = 0;
+    fail_at = at;
+    auto f = [&](int w, long long) { return hipMemcpyAsync(x.pin[w], a.data(), 1000, 0, nullptr); };
+    if (gpx::Xfer::run(4, 9, nullptr, f) != hipErrorUnknown) return 2;
+    if (waited < last_copy) return 3;
+  }
+  x.release();
+}
+"""
+
+
+def test_transfer_without_threads_and_after_an_error(tmp_path):
+    """A worker that cannot be started leaves its chunks to the others, and no
+    exception crosses the C entry; a transfer that fails returns when nothing
+    it has queued uses its buffers any more."""
+    run(tmp_path, XFER_STUB, XFER)
