@@ -35,6 +35,7 @@
 #include "gp_device.h"
 #include "gp_io.h"
 #include "gp_mlp.h"
+#include "gp_order.h"
 #include "gp_scan.h"
 #include "gp_xfer.h"
 
@@ -170,23 +171,8 @@ __device__ __forceinline__ int block_index(int xcd_remap) {
   return (b & 7) * per + (b >> 3);
 }
 
-// The advance's workgroup order in the reference's cell order (x fastest, then
-// y, then z): the particles of a z layer are cut into eight y blocks, one
-// for each XCD, and every XCD goes through its own y block layer by layer.
-// Layers are taken as equally full (the order is a permutation of the
-// workgroups whatever the particles do; how well the caches do depends on
-// it).  layers = 0: block_index.
-struct LayerMap {
-  int nb = 0;       // workgroups with work
-  int layers = 0;   // z layers of cells
-  int per = 0;      // workgroups launched for each (layer, y block), nb's share rounded up
-};
 __device__ __forceinline__ int layer_block(const LayerMap& lm, int xcd_remap) {
-  if (!lm.layers) return block_index(xcd_remap);
-  const int b = blockIdx.x, y = b & 7, t = b >> 3, j = t % lm.per, z = t / lm.per;
-  const long long k = 8ll * z + y, n = 8ll * lm.layers;
-  const int lo = (int)(k * lm.nb / n), hi = (int)((k + 1) * lm.nb / n);
-  return lo + j < hi ? lo + j : lm.nb;   // nb: nothing to do
+  return lm.layers ? layer_item(lm, blockIdx.x) : block_index(xcd_remap);
 }
 
 __device__ __forceinline__ long long node_index(int n4, int i, int j, int k) {
@@ -3530,16 +3516,9 @@ static void launch_advance_kernel(gp_ctx* ctx, hipStream_t st, const int* perm, 
     return;
   }
   unsigned nb = nblk(np);
-  // y blocks per XCD where a layer's y block fills four workgroups or more: at
-  // 8e6 particles on 512^3 (12 of them) the FP32 advance takes 2620 us against
-  // 2804 in plain order, at 1e6 on 256^3 (2.5) 344 against 338
   LayerMap lm;
-  if (!xcd && perm && perm != ctx->trav && nb >= 32u * (unsigned)ctx->g.nz) {
-    lm.nb = (int)nb;
-    lm.layers = ctx->g.nz;
-    lm.per = (int)((nb + 8u * ctx->g.nz - 1) / (8u * ctx->g.nz));
-    nb = 8u * (unsigned)lm.layers * (unsigned)lm.per;
-  }
+  if (!xcd && perm && perm != ctx->trav) lm = layer_map((int)nb, np, ctx->g.nbox, ctx->g.nz);
+  if (lm.layers) nb = (unsigned)layer_grid(lm);
   if (xcd) nb = (nb + 7) / 8 * 8;
   const dim3 gr(nb), bl(BLOCK);
 #define GP_ADV(FT, CT, S)                                                                        \

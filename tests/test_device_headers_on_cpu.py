@@ -180,3 +180,47 @@ def test_transfer_without_threads_and_after_an_error(tmp_path):
     exception crosses the C entry; a transfer that fails returns when nothing
     it has queued uses its buffers any more."""
     run(tmp_path, XFER_STUB, XFER)
+
+
+ORDER = r"""
+#include <cstdio>
+#include <vector>
+#include "gp_order.h"
+using namespace gp;
+int main() {
+  const int nzs[] = {1, 2, 3, 7, 20, 54, 244, 320};
+  for (int nz : nzs)
+    for (int nb = 1; nb < 40 * nz + 700; nb += nb < 300 ? 1 : 97) {
+      const int nbox = nz * nz * nz, np = 256 * nb - 17;
+      const LayerMap lm = layer_map(nb, np, nbox, nz);
+      const bool want = nb >= 32 * nz && np < 6 * nbox;
+      if ((lm.layers == nz) != want || (lm.layers != 0) != want) return 1;
+      LayerMap m;   // the order itself, also where the rule does not take it
+      m.nb = nb;
+      m.layers = nz;
+      m.per = (nb + 8 * nz - 1) / (8 * nz);
+      if (want && (lm.nb != m.nb || lm.per != m.per)) return 2;
+      std::vector<int> seen(nb + 1, 0);
+      for (int b = 0; b < layer_grid(m); ++b) {
+        const int i = layer_item(m, b);
+        if (i < 0 || i > nb) return 3;
+        seen[i]++;
+      }
+      for (int i = 0; i < nb; ++i)
+        if (seen[i] != 1) return 4;
+    }
+  // the largest products
+  LayerMap m;
+  m.nb = 8388607; m.layers = 1290; m.per = (m.nb + 8 * 1290 - 1) / (8 * 1290);
+  std::printf("%d\n", layer_item(m, layer_grid(m) - 8 * m.per + 7));
+}
+"""
+
+
+def test_layer_order_of_the_library(tmp_path):
+    """The advance's workgroup order as the library has it takes every
+    workgroup exactly once, and is on only where cells hold fewer than six
+    particles on average."""
+    out = run(tmp_path, HIP_STUB, ORDER)
+    nb, n = 8388607, 8 * 1290
+    assert int(out) == (n - 1) * nb // n
