@@ -1113,10 +1113,12 @@ __device__ __forceinline__ void min_image(const PState<VT>& p, int i, int j, dou
 constexpr int PF_STAGE = 1024;
 
 // GROUPED: several ensembles (gsort given), a variant of its own so that
-// the plain test keeps its registers.  DENSE: cells of a particle or more on
+// the plain test keeps its registers.  DENSE: cells of 1.5 particles or more on
 // average, whose further members are read three at a time (one trip to the
-// caches for three tests): 2e6 particles in 5 % by volume 610 -> 490 us; in
-// sparse cells (1e6 in 1e-3: 0.14 a cell) it took 84 us against 80.
+// caches for three tests): 2e6 particles in 5 % by volume 610 -> 490 us.  Both
+// filters, plain -> three at a time, at 0.14 particles a cell 102 -> 106 us,
+// 0.42 107 -> 112, 0.84 120 -> 124, 1.45 154.7 -> 155.1, 2.5 202 -> 193, 5.1
+// 284 -> 262, 13 519 -> 456 (1e6 particles; 2e5 the same way).
 template <bool GROUPED, bool DENSE = false>
 __global__ __launch_bounds__(BLOCK) void k_prefilter(
     CellGrid g, const float4* __restrict__ pos4, const int* __restrict__ sorted,
@@ -3798,7 +3800,8 @@ static int launch_contacts_filter(gp_ctx* ctx, bool list_lm, bool clear_bins = f
                        ctx->work, c + 1, ctx->work_cap, c + 11, ctx->d_err, np,
                        ctx->prm.xcd_remap);
   else
-    hipLaunchKernelGGL((np >= ctx->g.nbox ? k_prefilter<false, true> : k_prefilter<false, false>),
+    hipLaunchKernelGGL((2ll * np >= 3ll * ctx->g.nbox ? k_prefilter<false, true>
+                                                       : k_prefilter<false, false>),
                        dim3(xcd_grid(ctx, np)), dim3(BLOCK), 0, ctx->st,
                        ctx->g, ctx->pos4, ctx->sorted, ctx->csort, ctx->off, ctx->cnt,
                        (const int*)nullptr, ctx->prm.L, prefilter_tol(ctx), ctx->prm.prefilter,
