@@ -217,25 +217,16 @@ __device__ __noinline__ double enorm_scaled(double x0, double x1, double x2, int
   return sqrt(x3max * ((s2 / x3max) + (x3max * s3)));
 }
 
-constexpr double RDWARF = 3.834e-20, RGIANT = 1.304e19;
-
+// Sums of squares that are right to their rounding whatever the components:
+// far enough from the ends of the range that no square of a component that
+// matters has lost bits below 2^-1022 or overflowed.  Zero, infinities and
+// NaN are outside.
 constexpr unsigned high_word(double x) {
   return (unsigned)(__builtin_bit_cast(unsigned long long, x) >> 32);
 }
-// Intermediate magnitudes (RDWARF < |x| < RGIANT / 3) and zero, from the high
-// word without its sign, times two
-constexpr unsigned MID_LO = 2u * (high_word(RDWARF) + 1);
-constexpr unsigned MID_RANGE = 2u * high_word(RGIANT / 3.0) - MID_LO;
-__device__ __forceinline__ bool zero_or_mid(double x) {
-  return ((unsigned)__double2hiint(x) << 1) - MID_LO < MID_RANGE || x == 0.0;
-}
-// Sums of squares that are right whatever the components: none of them is as
-// large as RGIANT / 3, and those at or below RDWARF, however small, are a
-// part of 2^-59 or less.  Infinities and NaN are outside.
-constexpr unsigned SUM_LO = high_word(RDWARF * RDWARF * 0x1p60) + 1;
-constexpr unsigned SUM_RANGE = high_word(RGIANT / 3.0 * (RGIANT / 3.0)) - SUM_LO;
-__device__ __forceinline__ bool plain_sum(double sq) {
-  return (unsigned)__double2hiint(sq) - SUM_LO < SUM_RANGE;
+constexpr unsigned SUM_LO = high_word(0x1p-900), SUM_RANGE = high_word(0x1p1000) - SUM_LO;
+__device__ __forceinline__ unsigned sum_word(double sq) {
+  return (unsigned)__double2hiint(sq) - SUM_LO;
 }
 
 // x x as a number of its own, never inside a fused sum
@@ -248,28 +239,23 @@ __device__ __forceinline__ double fma2(double a, double b, double c, double d, d
   return __builtin_fma(a, b, __builtin_fma(c, d, e));
 }
 
-// enorm.  When every component is zero or of intermediate magnitude
-// (rdwarf < |x| < rgiant / N) MINPACK's sums reduce to s1 = s3 = x3max = 0
-// and the result to sqrt(s2), s2 the plain sum of squares; smaller components
-// beside a sum of squares 2^60 times theirs change it by less than its
-// rounding (bodies of revolution about a common axis, spheres above all, have
-// such residues of zeros in most of their norms).  FAST: only that, noting in
-// `far` where it was not right; else the others go to enorm_scaled.  The
-// sum's roundings are fixed: component R is squared first.
+// enorm.  MINPACK sums the components in three ranges so that no square
+// underflows or overflows; the root of the plain sum is the same number to
+// its rounding wherever the sum is within 2^-900 to 2^1000 (and the same bits
+// where every component is zero or in its middle range, 3.834e-20 to
+// 1.304e19 / n).  FAST: only that, keeping in `far` the sum_word furthest
+// out; else other sums go to enorm_scaled.  The sum's roundings are fixed:
+// component R is squared first.
 template <bool FAST, int N, int R = 1>
-__device__ __forceinline__ double enorm(const double* x, bool& far) {
+__device__ __forceinline__ double enorm(const double* x, unsigned& far) {
   double sq = __builtin_fma(x[1 - R], x[1 - R], sqr(x[R]));
   if (N > 2) sq = __builtin_fma(x[2], x[2], sq);
-  bool plain = plain_sum(sq);
-  if (!plain) {
-    plain = zero_or_mid(x[0]) & zero_or_mid(x[1]);
-    if (N > 2) plain &= zero_or_mid(x[2]);
-  }
   if (FAST) {
-    far |= !plain;
+    far = max(far, sum_word(sq));
     return sqrt(sq);
   }
-  return plain ? sqrt(sq) : enorm_scaled(x[0], x[1], N > 2 ? x[2] : 0.0, N);
+  return sum_word(sq) < SUM_RANGE ? sqrt(sq)
+                                  : enorm_scaled(x[0], x[1], N > 2 ? x[2] : 0.0, N);
 }
 
 constexpr double EPSMCH = 2.220446049250313e-16;
@@ -278,7 +264,7 @@ constexpr double DWARF = 2.2250738585072014e-308;
 // qrfac with column pivoting (minpack_reduc.f90:1007-1120), m = 3, n = 2
 template <bool FAST>
 __device__ __forceinline__ void qrfac32(double a[6], int ipvt[2], double rdiag[2],
-                                        double acnorm[2], double wa[2], bool& far) {
+                                        double acnorm[2], double wa[2], unsigned& far) {
   for (int j = 0; j < 2; ++j) {
     acnorm[j] = enorm<FAST, 3>(a + 3 * j, far);
     rdiag[j] = acnorm[j];
@@ -388,7 +374,7 @@ __device__ __forceinline__ void qrsolv2(double r[6], const int ipvt[2], const do
 template <bool FAST>
 __device__ __forceinline__ void lmpar2(double r[6], const int ipvt[2], const double diag[2],
                                        const double qtb[2], double delta, double& par,
-                                       double x[2], double sdiag[2], bool& far) {
+                                       double x[2], double sdiag[2], unsigned& far) {
   const double p1 = 0.1, p001 = 1.0e-3;
   double wa1[2], wa2[2];
   int nsing = 2;
@@ -457,7 +443,7 @@ struct LmState {
 template <bool FAST>
 __device__ __forceinline__ void lm_factor(const ContactPair& cp, const Jet& s,
                                           const double fvec[3], bool first, LmState& t,
-                                          bool& far) {
+                                          unsigned& far) {
   double fjac[6], wa1[2], wa2[2], wa3[2], wa4[3];
   int ipvt[2];
   fcn_j(cp, s, fjac);
@@ -518,7 +504,7 @@ __device__ __forceinline__ bool lm_run(const ContactPair& cp, LmState& s, int ma
   const double p1 = 0.1, p5 = 0.5, p25 = 0.25, p75 = 0.75, p0001 = 1.0e-4;
   for (;;) {
     LmState t = s;
-    bool far = false;
+    unsigned far = 0;
     const bool first = s.nfev == 0;
     const int ipvt[2] = {t.swapped, 1 - t.swapped};
     double fjac[6] = {t.r[0], 0.0, 0.0, t.r[1], t.r[2], 0.0};
@@ -581,7 +567,7 @@ __device__ __forceinline__ bool lm_run(const ContactPair& cp, LmState& s, int ma
       }
     }
     if (t.info == 0 && accept) lm_factor<FAST>(cp, trial, wa4, first, t, far);
-    if (FAST && far) return false;
+    if (FAST && far >= SUM_RANGE) return false;
     s = t;
     if (s.info != 0) return true;
   }
@@ -599,13 +585,15 @@ __device__ __noinline__ void lm_rest(const ContactPair* cp, LmState* s, int maxf
 // below 300 only for a network-seeded first attempt.
 // The solve is a serial chain of some 2000 instructions an evaluation.  Its
 // 13 norms each had a branch to the scaled sums, a call in the loop, for
-// vectors that hardly ever come (every component tiny: of 4000 pairs at most
-// one, whatever the bodies' symmetry): the loop runs without them, and a
-// solve that meets one goes on from there out of line.  Launches of 16 to 5e5
-// solves: 70 -> 64 us (1e4 particles on 64^3), 200 -> 177 (123457, four
-// points), 369 -> 326 (1e6 mixed), 2840 -> 2290 (2e6 in 5 % by volume); 2e6
-// spheres in 5 % by volume 2580 -> 2020 (2650 when a residue of zero in one
-// component counted as such a vector: 96 % of the solves left the loop).
+// vectors that hardly ever come: the loop runs without them, and a solve that
+// meets one goes on from there out of line.  Which ones is decided by the sum
+// of squares alone: by the components (each in MINPACK's middle range, or
+// zero) it took two instructions a component, and spheres, whose Jacobians
+// have rounding residues of zeros in most columns, left the loop in 96 % of
+// their solves.  Launches, branch -> by components -> by the sum: 16 solves
+// (1e4 particles on 64^3, 100^3) 70 -> 63.7 -> 60.6 us; a step's solve stage,
+// 4.4e3 solves 467 -> 406 -> 377, 5.2e5 2590 -> 2150 -> 1990, 4e5 of spheres
+// 2580 -> 2630 -> 2010.
 __device__ int lm_solve(const ContactPair& cp, double x[2], int* info_out, Jet& cur,
                         int maxfev = 300) {
   LmState s{};
