@@ -1847,9 +1847,9 @@ __global__ __launch_bounds__(GREEDY_BLOCK) void k_greedy_rounds(
 // every round in one workgroup, one launch instead of four, where the last
 // count of the present particles' solves (which bounds the contacts and,
 // unlike them, does not depend on the velocities) is at most GREEDY_FEW; any
-// number is right, but 1.6e5 contacts take 6.5 ms instead of 4.3.  A new set of
-// particles starts unknown, and a captured graph goes when a count read back
-// is larger.
+// number is right, but 1.6e5 contacts take 6.5 ms instead of 4.3.  Another
+// number of particles or other species start unknown, and a captured graph
+// goes when a count read back is larger.
 // Bound by the launches: 1e4 particles on 64^3 (some ten contacts) 13.7 us in
 // four launches, 5.0 us in one (a pass of 64 steps 13.2 -> 12.1 ms).
 // Thousands of contacts want more than one workgroup.
@@ -3184,7 +3184,9 @@ int gp_set_particles(gp_ctx* ctx, int np, const double* state, const int* specie
   hipStreamSynchronize(ctx->st2);
   hipStreamSynchronize(ctx->st3);
   drop_graph(ctx);
-  ctx->solved = ctx->nlm_known = false;
+  // as many particles of the same species, in one ensemble before and after:
+  // taken to be as dense (a host code that hands its particles over each step)
+  if (np != ctx->np || ctx->ngroups > 1) ctx->solved = ctx->nlm_known = false;
   ctx->contacts_valid = false;
   ctx->lists_sized = false;
   ctx->pipe_prev = false;
