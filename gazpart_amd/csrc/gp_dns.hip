@@ -769,6 +769,12 @@ struct Ran1 {
 
 using namespace gpdns;
 
+// the forcing of several steps goes to the device at once: at most FORCE_STEPS,
+// and FORCE_BYTES of amplitudes unless one step has more (a band of all modes:
+// 3 GB at 512^3)
+constexpr int FORCE_STEPS = 16;
+constexpr size_t FORCE_BYTES = (size_t)4 << 20;
+
 struct gp_dns {
   gp_dns_params prm{};
   Grid g{};
@@ -794,7 +800,8 @@ struct gp_dns {
   std::vector<double> fkf;
   std::vector<double> famp;    // [3][nf][2]
   int* fmap = nullptr;
-  double2* fdev = nullptr;     // amplitudes of FORCE_STEPS steps
+  int fsteps = FORCE_STEPS;    // steps whose forcing goes to the device at once
+  double2* fdev = nullptr;     // their amplitudes
   double* fpin = nullptr;      // and their page-locked staging
   Ran1 rng;
   std::string err;
@@ -843,7 +850,6 @@ int c2r(gp_dns* d, double2* in, double* out) {
 // ADV_FORCING (adv_forcing.f90:33-125) on the host for the next ns steps (it
 // depends on nothing but its own sequence): one copy to the device for all
 // of them.  The stream is idle here (gp_dns_step).
-constexpr int FORCE_STEPS = 16;
 
 int advance_forcing(gp_dns* d, int ns) {
   const int nf = (int)d->fmode.size();
@@ -1094,7 +1100,9 @@ int gp_dns_create(const gp_dns_params* p, gp_dns** out) {
     const size_t nf = d->fmode.size();
     d->famp.assign(3 * nf * 2, 0.0);   // INITIATION_FORCING_NEW: F = 0
     d->rng.idum = p->seed;
-    const size_t fb = std::max<size_t>(3 * nf, 1) * FORCE_STEPS * sizeof(double2);
+    const size_t one = std::max<size_t>(3 * nf, 1) * sizeof(double2);
+    d->fsteps = (int)std::min<size_t>(FORCE_STEPS, std::max<size_t>(FORCE_BYTES / one, 1));
+    const size_t fb = one * (size_t)d->fsteps;
     if (hipMalloc((void**)&d->fmap, nm * sizeof(int)) != hipSuccess ||
         hipMalloc((void**)&d->fdev, fb) != hipSuccess ||
         hipHostMalloc((void**)&d->fpin, fb) != hipSuccess)
@@ -1186,9 +1194,9 @@ int gp_dns_step(gp_dns* d, int nsteps) {
     d->err = "no velocity (gp_dns_set_velocity)";
     return GP_ERR_STATE;
   }
-  // in turns of FORCE_STEPS steps, whose forcing goes to the device at once
-  for (int s0 = 0; s0 < nsteps; s0 += FORCE_STEPS) {
-    const int ns = std::min(FORCE_STEPS, nsteps - s0);
+  // in turns of fsteps steps
+  for (int s0 = 0; s0 < nsteps; s0 += d->fsteps) {
+    const int ns = std::min(d->fsteps, nsteps - s0);
     int rc = advance_forcing(d, ns);
     for (int s = 0; s < ns && !rc; ++s)
       rc = one_step(d, d->fdev ? d->fdev + 3 * (size_t)s * d->fmode.size() : nullptr);
