@@ -275,9 +275,10 @@ def roofline(wl, res, scheme, cfg, launch, launch_fp64):
 # Peak evaluation rate of the contact solve, had every lane of every SIMD a
 # pair and the SIMDs issued without stalls: a wavefront of 64 solves takes
 # VALU_PER_EVAL VALU instructions per function evaluation (SQ counters on
-# the solve kernel: SQ_INSTS_VALU / evaluations per wavefront), FP64
+# the solve kernel: the slope of SQ_INSTS_VALU over the evaluations of 120
+# launches of one pair each), FP64
 # instructions issuing at one per 4 cycles on a SIMD (wave64 over 16 lanes)
-VALU_PER_EVAL = 1567.0
+VALU_PER_EVAL = 1157.0
 SIMDS = 1024
 CLOCK_HZ = 2.4e9
 

@@ -34,9 +34,13 @@
 //   k_fx_c2r     B -> u                                            2 F
 // 36 F in all, against 63 F for seven library transforms and separate
 // element-wise kernels.  Measured, us a step, library transforms -> these
-// passes: 32^3 123 -> 67, 64^3 184 -> 114, 100^3 477 -> 274, 128^3 709 -> 390,
-// 144^3 1064 -> 712, 192^3 2438 -> 1790, 256^3 6565 -> 3371 (36 F = 15.4 GB
-// with the padding, 4.6 TB/s), 320^3 12455 -> 9476.  (E = exp(-VISC |k|^2 DTIME), P the projection of
+// passes: 32^3 121 -> 63, 48^3 187 -> 125, 64^3 184 -> 111, 80^3 239 -> 195, 96^3
+// 378 -> 231, 100^3 415 -> 263, 128^3 691 -> 375, 144^3 1048 -> 714, 160^3 1291
+// -> 1010, 192^3 2435 -> 1712, 256^3 6500 -> 3355 (36 F = 15.4 GB with the
+// padding, 4.6 TB/s), 320^3 12524 -> 8717, 384^3 24650 -> 14490, 512^3 53460 ->
+// 31100.  Error of the velocity against 80-bit arithmetic, rms: 64^3 after 40
+// steps 8.4e-15 -> 6.8e-15, 128^3 after 16 6.5e-15 -> 2.4e-15, 256^3 after 3
+// 1.4e-15 -> 7.9e-16.  (E = exp(-VISC |k|^2 DTIME), P the projection of
 // NONLINEAR_TERMS's RHS assembly.)
 //
 // Lengths without a plan in gp_fft.h take rocFFT's batched transforms and
