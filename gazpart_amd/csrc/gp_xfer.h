@@ -46,9 +46,12 @@ struct Xfer {
     }
   }
 
-  // buffers of the first n workers (device ones on request); the transfers
-  // that used the old ones are complete
-  hipError_t reserve(int n, size_t bytes, bool device) {
+  // buffers of the first n workers (device ones on request), of bytes or more
+  // (at most XFER_CHUNK: lists that grow from call to call do not allocate
+  // each time); the transfers that used the old ones are complete
+  hipError_t reserve(int n, size_t least, bool device) {
+    size_t bytes = 4096;
+    while (bytes < least) bytes *= 2;
     for (int b = 0; b < n; ++b) {
       hipError_t e;
       if (!ev[b] && (e = hipEventCreateWithFlags(&ev[b], hipEventDisableTiming)) != hipSuccess)

@@ -115,14 +115,20 @@ typedef void* hipEvent_t;
 typedef void* hipStream_t;
 enum { hipSuccess = 0, hipErrorUnknown = 999 };
 enum { hipEventDisableTiming, hipMemcpyDeviceToHost, hipMemcpyHostToDevice };
-inline std::atomic<int> calls{0}, copies{0}, last_copy{0}, waited{0}, fail_at{-1};
+inline std::atomic<int> calls{0}, copies{0}, last_copy{0}, waited{0}, fail_at{-1}, allocs{0};
+inline std::atomic<size_t> largest{0};
 inline hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
 inline hipError_t hipSetDevice(int) { return hipSuccess; }
 inline hipError_t hipEventCreateWithFlags(hipEvent_t* e, int) { *e = e; return hipSuccess; }
 inline hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
 inline hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
 inline hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
-inline hipError_t hipHostMalloc(void** p, size_t n) { *p = std::malloc(n); return hipSuccess; }
+inline hipError_t hipHostMalloc(void** p, size_t n) {
+  ++allocs;
+  if (n > largest) largest = n;
+  *p = std::malloc(n);
+  return hipSuccess;
+}
 inline hipError_t hipHostFree(void* p) { std::free(p); return hipSuccess; }
 inline hipError_t hipMalloc(void** p, size_t n) { return hipHostMalloc(p, n); }
 inline hipError_t hipFree(void* p) { return hipHostFree(p); }
@@ -171,6 +177,16 @@ int main() {
     if (waited < last_copy) return 3;
   }
   x.release();
+  // a list that grows by a few entries a call, to the largest chunk and past it
+  gpx::Xfer y;
+  fail_at = -1;
+  allocs = 0;
+  largest = 0;
+  for (size_t m = 100; m < n; m += m < 200000 ? 4100 : 99991)
+    if (y.d2h(b.data(), a.data(), m, nullptr) != hipSuccess) return 4;
+  y.release();
+  // 4 KB to 4 MB in doublings, once a worker
+  if (allocs > 11 * gpx::XFER_WORKERS || largest > gpx::XFER_CHUNK) return 5;
 }
 """
 
@@ -178,7 +194,8 @@ int main() {
 def test_transfer_without_threads_and_after_an_error(tmp_path):
     """A worker that cannot be started leaves its chunks to the others, and no
     exception crosses the C entry; a transfer that fails returns when nothing
-    it has queued uses its buffers any more."""
+    it has queued uses its buffers any more; buffers grow by doubling, to a chunk at
+    most."""
     run(tmp_path, XFER_STUB, XFER)
 
 
