@@ -46,29 +46,32 @@ struct Xfer {
     }
   }
 
-  // buffers of the first n workers (device ones on request), of bytes or more
-  // (at most XFER_CHUNK: lists that grow from call to call do not allocate
-  // each time); the transfers that used the old ones are complete
-  hipError_t reserve(int n, size_t least, bool device) {
-    size_t bytes = 4096;
-    while (bytes < least) bytes *= 2;
+  // buffers of the first n workers (device ones on request); one that is too
+  // small is followed by one of twice its size or more, up to XFER_CHUNK, so
+  // that lists that grow from call to call do not allocate each time (the
+  // first is as large as asked: page-locking takes 0.35 ms a MB).  The
+  // transfers that used the old ones are complete
+  hipError_t reserve(int n, size_t bytes, bool device) {
+    auto size = [&](size_t had) { return std::max(bytes, std::min(XFER_CHUNK, 2 * had)); };
     for (int b = 0; b < n; ++b) {
       hipError_t e;
       if (!ev[b] && (e = hipEventCreateWithFlags(&ev[b], hipEventDisableTiming)) != hipSuccess)
         return e;
       if (pin_n[b] < bytes) {
+        const size_t m = size(pin_n[b]);
         if (pin[b]) (void)hipHostFree(pin[b]);
         pin[b] = nullptr;
         pin_n[b] = 0;
-        if ((e = hipHostMalloc((void**)&pin[b], bytes)) != hipSuccess) return e;
-        pin_n[b] = bytes;
+        if ((e = hipHostMalloc((void**)&pin[b], m)) != hipSuccess) return e;
+        pin_n[b] = m;
       }
       if (device && dev_n[b] < bytes) {
+        const size_t m = size(dev_n[b]);
         if (dev[b]) (void)hipFree(dev[b]);
         dev[b] = nullptr;
         dev_n[b] = 0;
-        if ((e = hipMalloc((void**)&dev[b], bytes)) != hipSuccess) return e;
-        dev_n[b] = bytes;
+        if ((e = hipMalloc((void**)&dev[b], m)) != hipSuccess) return e;
+        dev_n[b] = m;
       }
     }
     return hipSuccess;
